@@ -21,15 +21,23 @@
 // puts a (src, dst) pair in one workgroup for the co-occurrence counts).  Lane s
 // loads ring slot s (with its feature row when the row is at most 64 bytes, in
 // the same memory round trip) and the node's write position.  Ranking:
-//   * fast path (no CSR candidates): a ring is written oldest-to-newest from slot
-//     write_pos % B on, so when the filled slots are exactly the last ones in that
-//     write order and their times strictly increase along it, a candidate's rank
-//     is its write-order distance from the oldest filled slot (one shuffle and
-//     two ballots verify the premise);
-//   * otherwise the candidates go to an LDS list (CSR window first, then ring
-//     slots) and each is ranked by counting earlier (time, index) entries.
-// The lane holding a selected candidate writes its id / time / mask at output
-// position K - V + rank - drop; feature rows then move to their positions by
+//   * ring: slots are written oldest-to-newest from slot write_pos % B on, so
+//     when the filled slots are exactly the last ones in that write order and
+//     their times never decrease along it, a valid slot's rank among the valid
+//     slots is its write-order distance from the oldest filled slot (one shuffle
+//     and two ballots verify the premise); otherwise it is counted over the
+//     ring's times in LDS;
+//   * CSR and ring: the CSR window ends where a search of the node's times says,
+//     or at its last entry when that is before the query; when that entry is not
+//     after the oldest valid slot, the slots take the last output positions and
+//     the window's end the ones before them, each lane loading the entry of its
+//     own position.  Otherwise the two are merged through LDS.  (Before, every
+//     query with CSR entries staged K + B candidates and counted each against all
+//     others, in every wave that shares the query: 200 events, K = 32, B = 64,
+//     172-d rows with co-occurrence took 25.1 us, 16.0 now; 4,000 events with
+//     32-byte rows 54.1, 36.8.)
+// The lane holding a selected candidate writes its id / time / mask at its output
+// position; feature rows then move to their positions by
 // lane shuffles (small rows) or 16-byte loads/stores spread over the wave, and
 // the K x d_t encodings stream out as float4 nontemporal stores with the pad
 // rows (DyGFormer dt mode) written as zeros without evaluating a cosine.  The
@@ -105,8 +113,7 @@ struct Params {
   // LDS layout: weights (te_bytes), then one wave_bytes region per wavefront
   int te_bytes;
   int wave_bytes;
-  int cand_cap;
-  int off_cid, off_code, off_pcode, off_pdt, off_pid, off_pt, off_pe, off_tab;
+  int off_ct, off_cid, off_pcode, off_pdt, off_pid, off_pt, off_pe, off_tab;
   // work decomposition: m queries per wavefront in sub-groups of 2^lg_bp lanes
   int m, lg_bp;
   // FastDiv multipliers of K, d_t / 4, d_t and nch
@@ -517,14 +524,16 @@ __device__ __forceinline__ void co_occurrence_pair(const Params& P, int64_t g, i
 // kernel, where forcing 8 capped the scalar registers and spilled them into their
 // own code (the tiled one: 8.56 -> 7.74 us on C1 and 367 -> 356 us on C4 without
 // it), while the 7 the registers allow still hold their grids.
-template <int VEC, int NREG, bool TILES>
-constexpr int kWavesPerEu = NREG > 0 || (TILES && VEC == 16) ? 1 : 8;
+template <int VEC, int NREG, bool TILES, bool CSR>
+constexpr int kWavesPerEu = CSR || NREG > 0 || (TILES && VEC == 16) ? 1 : 8;
 
 // TILES: the launch's plan mode is TGX_PLAN_TILES (no event or list plan, so no
 // co-occurrence); that copy of the kernel carries none of their code, which
-// shortens its start-up
-template <int VEC, int NREG, bool TILES>
-__global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<VEC, NREG, TILES>)))
+// shortens its start-up.
+// CSR: the launch reads a frozen CSR (with or without a ring beside it); the copies
+// without it carry none of that code.
+template <int VEC, int NREG, bool TILES, bool CSR>
+__global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<VEC, NREG, TILES, CSR>)))
 void recent_fused(Params P) {
   using VT = typename Vec<VEC>::T;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -539,7 +548,6 @@ void recent_fused(Params P) {
   const int64_t g = static_cast<int64_t>(blockIdx.x) - P.plan_blocks;
   const int K = P.K;
   const int B = P.B;
-  const int C = P.cand_cap;
   const int m = P.m;
   const int lg = P.lg_bp;
   const int Bp = 1 << lg;
@@ -556,9 +564,9 @@ void recent_fused(Params P) {
   }
   __syncthreads();
   uint8_t* wb = smem + P.te_bytes + static_cast<size_t>(wv) * P.wave_bytes;
-  double* ct = reinterpret_cast<double*>(wb);                       // [m][C] candidates
+  double* rl = reinterpret_cast<double*>(wb);                       // [64] ring times (with a ring)
+  double* ct = reinterpret_cast<double*>(wb + P.off_ct);           // [m][K] CSR candidates (with a ring and a CSR)
   int32_t* cid = reinterpret_cast<int32_t*>(wb + P.off_cid);
-  int32_t* ccode = reinterpret_cast<int32_t*>(wb + P.off_code);
   int32_t* pcode = reinterpret_cast<int32_t*>(wb + P.off_pcode);  // [m][K] slot, B + CSR index, -1
   float* pdt = reinterpret_cast<float*>(wb + P.off_pdt);           // [m][K] dt
   int32_t* pid = reinterpret_cast<int32_t*>(wb + P.off_pid);       // [m][K] id
@@ -590,6 +598,15 @@ void recent_fused(Params P) {
   const int64_t ur = node < 0 ? 0 : node;
   const bool live = q >= 0 && qvalid && !bad;
 
+  // ---- the node's CSR range (a padding node's is empty), in the ring loads' round trip ----
+  int64_t s0 = 0, s1 = 0;
+  if constexpr (CSR) {
+    if (live && node >= 0) {
+      s0 = P.c_off[node];
+      s1 = P.c_off[node + 1];
+    }
+  }
+
   // ---- ring slot sl of query h, its feature row (NREG > 0) and write position ----
   int32_t rid = -1;
   double rt = 0.0;
@@ -615,41 +632,60 @@ void recent_fused(Params P) {
     }
   }
 
-  // ---- CSR windows: a 64-ary search per query of the wave, all lanes ----
-  int ncsr = 0;
-  int64_t cbase = 0;
-  if (P.has_csr) {
-    for (int hh = 0; hh < m; ++hh) {
-      const int64_t nh = __shfl(node, hh << lg);
-      const double th = __shfl(qt, hh << lg);
-      const int lh = __shfl(static_cast<int>(live), hh << lg);
-      if (lh && nh >= 0) {
-        const int64_t s0 = P.c_off[nh];
-        const int64_t s1 = P.c_off[nh + 1];
-        const int64_t cnt = wave_lower_bound<TILES>(P.c_times, s0, s1, th, lane) - s0;
-        const int take = static_cast<int>(cnt < K ? cnt : K);
-        if (h == hh) {
-          ncsr = take;
-          cbase = s0 + cnt - take;
-        }
-      }
-    }
-    for (int j = sl; j < ncsr; j += Bp) {
-      ct[h * C + j] = P.c_times[cbase + j];
-      cid[h * C + j] = P.c_ids[cbase + j];
-      ccode[h * C + j] = B + j;
-    }
-  }
   const bool v = live && sl < B && rid != -1 && rt < qt;
   const uint64_t mine = (__ballot(v) >> (h << lg)) & submask;
-  const int ncand = ncsr + __popcll(mine);
-  const int V = ncand < K ? ncand : K;
-  const int drop = ncand - V;
-  if (sl == 0) {
-    tq[h] = q;
-    tur[h] = ur;
-    tcb[h] = cbase;
+  const int nring = __popcll(mine);
+
+  // ---- CSR window [s0, e) of entries before the query time ----
+  // Lane sl first loads the entry that position sl gets when every CSR entry of
+  // the node is before the query and before the valid ring slots (the usual case
+  // once the graph is frozen): e = s1, the valid slots take the last positions
+  // and the window's end the ones before them.  The window's last time and, for a
+  // query that may fall inside the window (not after the CSR's largest time), the
+  // search's first Bp-ary round go out with it.
+  int64_t e = s1;
+  double tlast = 0.0, ct0 = 0.0;
+  int32_t cid0 = -1;
+  bool have0 = false;
+  if constexpr (CSR) {
+    auto load_first = [&]() {
+      const int64_t x = e - K + nring + sl;
+      have0 = sl < K - nring && x >= s0 && x < e;
+      if (have0) {
+        ct0 = P.c_times[x];
+        cid0 = P.c_ids[x];
+      }
+    };
+    if (s1 > s0) tlast = P.c_times[s1 - 1];
+    load_first();
+    const int64_t wlen = s1 - s0;
+    const bool probing = wlen > Bp && qt <= P.c_tmax;
+    const int64_t step = probing ? (wlen + Bp - 1) >> lg : 0;
+    double tp = 0.0;
+    if (probing) {
+      const int64_t pos = s0 + (sl + 1) * step - 1;
+      tp = P.c_times[pos < s1 ? pos : s1 - 1];
+    }
+    const bool inside = s1 > s0 && !(tlast < qt);  // NaN times sort last
+    if (__ballot(inside) != 0) {  // wave-uniform
+      const uint64_t below = (__ballot(probing && tp < qt) >> (h << lg)) & submask;
+      int64_t lo = s0, hi = s1;
+      if (probing) {
+        const int64_t c = __popcll(below);
+        const int64_t nl = s0 + c * step;
+        const int64_t pc = s0 + (c + 1) * step - 1;
+        lo = nl < s1 ? nl : s1;
+        hi = pc < s1 ? pc : s1;
+      }
+      const int64_t end = subgroup_lower_bound(P.c_times, lo, hi, qt, inside, sl, h, lg);
+      if (inside) {
+        e = end;
+        if (e > s0) tlast = P.c_times[e - 1];
+        load_first();
+      }
+    }
   }
+  const int ncsr = CSR ? static_cast<int>(e - s0 < K ? e - s0 : K) : 0;
 
   // ---- rank into LDS positions ----
   bool lane_big = false;
@@ -662,57 +698,106 @@ void recent_fused(Params P) {
     pid[pp] = id;
     lane_big |= (!dyg || code >= 0) && !(fabsf(dt) < P.te_dt_small);
   };
-  // fast path: no CSR candidates, and the filled slots are the newest ones in
-  // write order (oldest = slot write_pos % B) with strictly increasing times;
-  // then a candidate's rank is its write-order distance from the oldest filled slot
-  bool broken = true;
+  // A valid slot's rank among the valid slots (time, then slot).  When the filled
+  // slots are the newest ones in write order (oldest = slot write_pos % B) with
+  // times that never decrease along it (equal times only where the slot grows
+  // too), the rank is the write-order distance from the oldest filled slot;
+  // otherwise it is counted over the ring's times in LDS (NaN for a slot that is
+  // not valid: it compares false), two float64 compares per pair.
   int order = 0;
-  const bool try_fast = live && ncsr == 0 && B > 0 && P.r_wp != nullptr;
-  if (try_fast) {
+  bool broken = true;
+  const bool try_sorted = live && B > 0 && P.r_wp != nullptr;
+  if (try_sorted) {
     const int w = P.b_pow2 ? static_cast<int>(wp & (B - 1)) : static_cast<int>(wp % B);
     order = sl - w < 0 ? sl - w + B : sl - w;
     const uint64_t filled = (__ballot(sl < B && rid != -1) >> (h << lg)) & submask;
     const int empty = B - __popcll(filled);
     const int nxt = sl + 1 == B ? 0 : sl + 1;
     const double tn = __shfl(rt, (h << lg) + nxt);
-    broken = sl < B && (((rid != -1) != (order >= empty)) || (rid != -1 && order < B - 1 && !(rt < tn)));
+    broken = sl < B && (((rid != -1) != (order >= empty)) ||
+                        (rid != -1 && order < B - 1 && !(nxt != 0 ? rt <= tn : rt < tn)));
     order -= empty;
   }
-  const bool fast = try_fast && ((__ballot(broken) >> (h << lg)) & submask) == 0;
-  if (q >= 0) {
-    if (fast) {
-      if (v && order >= drop) emit(K - V + (order - drop), rid, rt, sl);
-    } else if (v) {
-      const int at = h * C + ncsr + __popcll(mine & ((uint64_t(1) << sl) - 1));
-      ct[at] = rt;
-      cid[at] = rid;
-      ccode[at] = sl;
-    }
-  }
-  wave_sync();
-  if (q >= 0) {
-    if (!fast) {
-      // counting rank by (time, CSR-before-ring, candidate index).  The CSR
-      // window is time-ascending with ties in CSR order, so CSR entry c has
-      // exactly c such predecessors among the CSR entries and only the ring
-      // candidates need counting; a ring candidate counts them all
-      for (int c = sl; c < ncand; c += Bp) {
-        const double tc = ct[h * C + c];
-        int r = c < ncsr ? c : 0;
-        for (int c0 = c < ncsr ? ncsr : 0; c0 < ncand; c0 += 4) {
+  const bool sorted = try_sorted && ((__ballot(broken) >> (h << lg)) & submask) == 0;
+  if (__ballot(nring > 0 && !sorted) != 0) {  // wave-uniform
+    rl[lane] = v ? rt : __builtin_nan("");
+    wave_sync();
+    int r = 0;
+    const double* row = rl + (h << lg);
+    for (int c0 = 0; c0 < B; c0 += 4) {  // the row holds Bp >= 16 entries
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int c2 = c0 + u;
-            if (c2 < ncand) {
-              const double t2 = ct[h * C + c2];
-              r += (t2 < tc) || (t2 == tc && c2 < c);
-            }
-          }
-        }
-        if (r >= drop) emit(K - V + (r - drop), cid[h * C + c], tc, ccode[h * C + c]);
+      for (int u = 0; u < 4; ++u) {
+        const double t2 = row[c0 + u];
+        r += (t2 < rt) || (t2 == rt && c0 + u < sl);
       }
     }
-    for (int p = sl; p < K - V; p += Bp) emit(p, -1, 0.0, -1);
+    if (!sorted) order = r;
+  }
+  // With a CSR whose last candidate is not after the oldest valid slot (equal times
+  // keep CSR-before-ring), the valid slots follow the CSR entries; otherwise the
+  // two merge.  CSR entry of code B + j is entry cbase + j.
+  bool merge = false;
+  int64_t cbase = 0;
+  if constexpr (CSR) {
+    const uint64_t first = (__ballot(v && order == 0) >> (h << lg)) & submask;
+    const double told = __shfl(rt, (h << lg) + (first != 0 ? __builtin_ctzll(first) : 0));
+    merge = nring > 0 && ncsr > 0 && !(tlast <= told);
+    cbase = e - (merge ? ncsr : K - nring);
+    if (__ballot(merge) != 0) {  // wave-uniform
+      rl[lane] = v ? rt : __builtin_nan("");
+      if (merge)
+        for (int j = sl; j < ncsr; j += Bp) {
+          ct[h * K + j] = P.c_times[cbase + j];
+          cid[h * K + j] = P.c_ids[cbase + j];
+        }
+      wave_sync();
+    }
+  }
+  if (sl == 0) {
+    tq[h] = q;
+    tur[h] = ur;
+    if constexpr (CSR) tcb[h] = cbase;
+  }
+  if (q >= 0) {
+    if (CSR && merge) {
+      // a CSR entry follows the CSR entries before it and the slots with a smaller
+      // time; a slot the slots before it and the CSR entries up to its time
+      const int ncand = ncsr + nring;
+      for (int j = sl; j < ncsr; j += Bp) {
+        const double tc = ct[h * K + j];
+        int r = j;
+        for (int c = 0; c < B; ++c) r += rl[(h << lg) + c] < tc;
+        if (K - ncand + r >= 0) emit(K - ncand + r, cid[h * K + j], tc, B + j);
+      }
+      if (v) {
+        int lo = 0, hi = ncsr;
+        while (lo < hi) {
+          const int mid = (lo + hi) >> 1;
+          if (ct[h * K + mid] <= rt)
+            lo = mid + 1;
+          else
+            hi = mid;
+        }
+        if (K - ncand + order + lo >= 0) emit(K - ncand + order + lo, rid, rt, sl);
+      }
+      for (int p = sl; p < K - ncand; p += Bp) emit(p, -1, 0.0, -1);
+    } else {
+      if (v && K - nring + order >= 0) emit(K - nring + order, rid, rt, sl);
+      for (int p = sl; p < K - nring; p += Bp) {
+        if constexpr (CSR) {
+          if (p != sl) {
+            have0 = cbase + p >= s0;
+            if (have0) {
+              ct0 = P.c_times[cbase + p];
+              cid0 = P.c_ids[cbase + p];
+            }
+          }
+          emit(p, have0 ? cid0 : -1, have0 ? ct0 : 0.0, have0 ? B + p : -1);
+        } else {
+          emit(p, -1, 0.0, -1);
+        }
+      }
+    }
   } else {
     for (int p = sl; p < K; p += Bp) {
       pcode[h * K + p] = -1;
@@ -739,12 +824,13 @@ void recent_fused(Params P) {
     for (int gp = lane; gp < np; gp += kWave) {
       const int hh = static_cast<int>(dk.div(gp));
       const int code = pcode[gp];
-      int64_t e = -1;
-      if (code >= 0 && code < B)
-        e = P.r_eids != nullptr ? P.r_eids[tur[hh] * B + code] : -1;
-      else if (code >= B)
-        e = P.c_eids != nullptr ? P.c_eids[tcb[hh] + (code - B)] : -1;
-      pe[gp] = e;
+      int64_t ev = -1;
+      if (code >= 0 && (!CSR || code < B)) {
+        ev = P.r_eids != nullptr ? P.r_eids[tur[hh] * B + code] : -1;
+      } else if constexpr (CSR) {
+        if (code >= B) ev = P.c_eids != nullptr ? P.c_eids[tcb[hh] + (code - B)] : -1;
+      }
+      pe[gp] = ev;
     }
   }
 
@@ -766,30 +852,38 @@ void recent_fused(Params P) {
     const FastDiv dv(nch, P.fd_c);
     VT* of = reinterpret_cast<VT*>(P.o_feats) + r0 * nch;
     if constexpr (NREG > 0) {
-      // ring rows come from the lanes that loaded them, CSR rows from memory;
-      // every lane takes part in every shuffle
-      for (int b0 = part * kWave; b0 < total; b0 += ostride) {
-        const int idx = b0 + lane;
-        int gp = 0, c = 0, code = -1, hh = 0;
-        if (idx < total) {
-          gp = static_cast<int>(dv.div(idx));
-          c = idx - gp * nch;
-          hh = static_cast<int>(dk.div(gp));
-          code = pcode[gp];
-        }
-        const int srcl = (code >= 0 && code < B) ? (hh << lg) + code : lane;
-        VT val = VT{};
+      // ring rows come from the lanes that loaded them, CSR rows from memory (kDepth
+      // of them loaded before the first is stored); every lane takes part in every
+      // shuffle
+      constexpr int kDepth = CSR ? kCopyDepth : 1;
+      for (int b0 = part * kWave; b0 < total; b0 += kDepth * ostride) {
+        VT v4[kDepth];
 #pragma unroll
-        for (int k = 0; k < NREG; ++k) {
-          const VT x = shfl_v(rows[k], srcl);
-          if (k == c) val = x;
+        for (int u = 0; u < kDepth; ++u) {
+          const int idx = b0 + u * ostride + lane;
+          int gp = 0, c = 0, code = -1, hh = 0;
+          if (idx < total) {
+            gp = static_cast<int>(dv.div(idx));
+            c = idx - gp * nch;
+            hh = static_cast<int>(dk.div(gp));
+            code = pcode[gp];
+          }
+          const int srcl = (code >= 0 && (!CSR || code < B)) ? (hh << lg) + code : lane;
+          VT val = VT{};
+#pragma unroll
+          for (int k = 0; k < NREG; ++k) {
+            const VT x = shfl_v(rows[k], srcl);
+            if (k == c) val = x;
+          }
+          if (code < 0) val = VT{};
+          if constexpr (CSR)
+            if (code >= B) val = reinterpret_cast<const VT*>(P.c_feats + (tcb[hh] + (code - B)) * P.row_bytes)[c];
+          v4[u] = val;
         }
-        if (idx < total) {
-          if (code < 0)
-            val = VT{};
-          else if (code >= B)
-            val = reinterpret_cast<const VT*>(P.c_feats + (tcb[hh] + (code - B)) * P.row_bytes)[c];
-          put<false>(of + idx, val);
+#pragma unroll
+        for (int u = 0; u < kDepth; ++u) {
+          const int idx = b0 + u * ostride + lane;
+          if (idx < total) put<false>(of + idx, v4[u]);
         }
       }
     } else {
@@ -810,8 +904,8 @@ void recent_fused(Params P) {
             const int hh = static_cast<int>(dk.div(gp));
             const int code = pcode[gp];
             if (code >= 0) {
-              const uint8_t* src = code < B ? P.r_feats + (tur[hh] * B + code) * P.row_bytes
-                                            : P.c_feats + (tcb[hh] + (code - B)) * P.row_bytes;
+              const uint8_t* src = !CSR || code < B ? P.r_feats + (tur[hh] * B + code) * P.row_bytes
+                                                    : P.c_feats + (tcb[hh] + (code - B)) * P.row_bytes;
               v4[u] = reinterpret_cast<const VT*>(src)[c];
             }
           }
@@ -839,8 +933,8 @@ void recent_fused(Params P) {
   };
   // Store order: with register-held rows there is nothing left to load, so the
   // bulk (the encodings) goes first; with large rows the row copy loads first,
-  // before any encoding store can hold its loads back in vmcnt.
-  if constexpr (NREG > 0) {
+  // before any encoding store can hold its loads back in vmcnt; and so with CSR rows.
+  if constexpr (NREG > 0 && !CSR) {
     store_te();
     store_feats();
   } else {
@@ -1477,13 +1571,14 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   P.status = a->status;
 
   const int K = a->k;
-  // LDS candidates: the CSR window and the ring slots.  A tiled launch without a
-  // ring runs csr_window or csr_split (below), which stage no candidates; the
-  // split rule sizes it as a recent_fused launch without them
+  // LDS of the rank: the ring's times, and with a CSR beside it K candidates (time
+  // and id).  A tiled launch without a ring runs csr_window or csr_split (below);
+  // the split rule sizes it as a recent_fused launch without them
   L.noring = ring == nullptr && mode == TGX_PLAN_TILES;
-  P.cand_cap = L.noring ? 0 : (P.has_csr ? K : 0) + P.B;
+  const int ring_lds = P.B > 0 ? kWave * 8 : 0;
+  const int cands = P.B > 0 && P.has_csr ? K : 0;
   auto wave_lds = [&](int m) {
-    return round16(m * P.cand_cap * 16) + round16(m * K * 4) * 3 + round16(m * K * 8) *
+    return ring_lds + round16(m * cands * 8) + round16(m * cands * 4) + round16(m * K * 4) * 3 + round16(m * K * 8) *
            (a->out_eids != nullptr ? 2 : 1) + round16(m * 24);
   };
   // Queries per wave.  Packing m = 64 / Bp queries into sub-groups of Bp >= B
@@ -1502,9 +1597,9 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   P.m = kWave >> lg;
   P.lg_bp = lg;
   P.te_bytes = 2 * round16(a->d_t * 4);
-  P.off_cid = round16(P.m * P.cand_cap * 8);
-  P.off_code = P.off_cid + round16(P.m * P.cand_cap * 4);
-  P.off_pcode = P.off_code + round16(P.m * P.cand_cap * 4);
+  P.off_ct = ring_lds;
+  P.off_cid = P.off_ct + round16(P.m * cands * 8);
+  P.off_pcode = P.off_cid + round16(P.m * cands * 4);
   P.off_pdt = P.off_pcode + round16(P.m * K * 4);
   P.off_pid = P.off_pdt + round16(P.m * K * 4);
   P.off_pt = P.off_pid + round16(P.m * K * 4);
@@ -1669,16 +1764,26 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
     return fail(TGX_ERR_ARG, "tgx_recent: timing_start and timing_stop must both be set or both NULL");
   static std::once_flag attr_once;
   std::call_once(attr_once, [] {
-    const void* fns[] = {reinterpret_cast<const void*>(recent_fused<16, 0, false>),
-                         reinterpret_cast<const void*>(recent_fused<16, 2, false>),
-                         reinterpret_cast<const void*>(recent_fused<16, 4, false>),
-                         reinterpret_cast<const void*>(recent_fused<4, 0, false>),
-                         reinterpret_cast<const void*>(recent_fused<2, 0, false>),
-                         reinterpret_cast<const void*>(recent_fused<16, 0, true>),
-                         reinterpret_cast<const void*>(recent_fused<16, 2, true>),
-                         reinterpret_cast<const void*>(recent_fused<16, 4, true>),
-                         reinterpret_cast<const void*>(recent_fused<4, 0, true>),
-                         reinterpret_cast<const void*>(recent_fused<2, 0, true>)};
+    const void* fns[] = {reinterpret_cast<const void*>(recent_fused<16, 0, false, false>),
+                         reinterpret_cast<const void*>(recent_fused<16, 2, false, false>),
+                         reinterpret_cast<const void*>(recent_fused<16, 4, false, false>),
+                         reinterpret_cast<const void*>(recent_fused<4, 0, false, false>),
+                         reinterpret_cast<const void*>(recent_fused<2, 0, false, false>),
+                         reinterpret_cast<const void*>(recent_fused<16, 0, false, true>),
+                         reinterpret_cast<const void*>(recent_fused<16, 2, false, true>),
+                         reinterpret_cast<const void*>(recent_fused<16, 4, false, true>),
+                         reinterpret_cast<const void*>(recent_fused<4, 0, false, true>),
+                         reinterpret_cast<const void*>(recent_fused<2, 0, false, true>),
+                         reinterpret_cast<const void*>(recent_fused<16, 0, true, false>),
+                         reinterpret_cast<const void*>(recent_fused<16, 2, true, false>),
+                         reinterpret_cast<const void*>(recent_fused<16, 4, true, false>),
+                         reinterpret_cast<const void*>(recent_fused<4, 0, true, false>),
+                         reinterpret_cast<const void*>(recent_fused<2, 0, true, false>),
+                         reinterpret_cast<const void*>(recent_fused<16, 0, true, true>),
+                         reinterpret_cast<const void*>(recent_fused<16, 2, true, true>),
+                         reinterpret_cast<const void*>(recent_fused<16, 4, true, true>),
+                         reinterpret_cast<const void*>(recent_fused<4, 0, true, true>),
+                         reinterpret_cast<const void*>(recent_fused<2, 0, true, true>)};
     for (const void* f : fns)
       (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     (void)hipGetLastError();
@@ -1691,14 +1796,23 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
     else
       hipLaunchKernelGGL(kernel, grid, block, L.lds, stream, L.P);
   };
-  // a tiled launch runs the kernel's TILES copy
+  // a tiled launch runs the kernel's TILES copy, one that reads CSR entries its CSR copy
   const bool tiles = L.P.plan_mode == TGX_PLAN_TILES;
-  auto pick = [&](auto k_tiles, auto k_other) {
-    if (tiles)
+  auto pick = [&](auto k_tiles, auto k_other, auto k_tiles_csr, auto k_other_csr) {
+    if (L.P.has_csr) {
+      if (tiles)
+        launch(k_tiles_csr);
+      else
+        launch(k_other_csr);
+    } else if (tiles) {
       launch(k_tiles);
-    else
+    } else {
       launch(k_other);
+    }
   };
+#define TGX_PICK(V, R) \
+  pick(recent_fused<V, R, true, false>, recent_fused<V, R, false, false>, recent_fused<V, R, true, true>, \
+       recent_fused<V, R, false, true>)
   if (L.window) {
     if (L.nreg == 2)
       launch(csr_window<2>);
@@ -1724,16 +1838,17 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
     }
   } else if (L.vec == 16) {
     if (L.nreg == 2)
-      pick(recent_fused<16, 2, true>, recent_fused<16, 2, false>);
+      TGX_PICK(16, 2);
     else if (L.nreg == 4)
-      pick(recent_fused<16, 4, true>, recent_fused<16, 4, false>);
+      TGX_PICK(16, 4);
     else
-      pick(recent_fused<16, 0, true>, recent_fused<16, 0, false>);
+      TGX_PICK(16, 0);
   } else if (L.vec == 4) {
-    pick(recent_fused<4, 0, true>, recent_fused<4, 0, false>);
+    TGX_PICK(4, 0);
   } else {
-    pick(recent_fused<2, 0, true>, recent_fused<2, 0, false>);
+    TGX_PICK(2, 0);
   }
+#undef TGX_PICK
   rc = check_launch(L.window ? "csr_window" : L.csr_split ? "csr_split" : "recent_fused");
   if (rc != TGX_OK || !L.want_plan || L.fuse_plan) return rc;
   return launch_plan(L.pl, stream);  // batches beyond the fused plan's size
