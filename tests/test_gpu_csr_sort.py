@@ -1,0 +1,65 @@
+"""The CSR build's sort, segments and row gather at the sizes where their shape
+changes, bit for bit against the oracle: runs of equal times and calls that start,
+end and lie inside and across the 2,048-event tiles of the segment search; sorts of
+one and several tiles per workgroup (2M keys, 2,048- and 4,096-key tiles); one to
+three digit passes; entry counts on both sides of the event-ordered gather (2^20)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import spec as O
+from tgengine_amd import TemporalGraph
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(N, d, cuts, src, dst, time, seed=0):
+    E = len(src)
+    feat = np.random.default_rng(seed).standard_normal((E, d)).astype(np.float32)
+    g = TemporalGraph(N, edge_feat_dim=d, device="cuda", track_edge_ids=True)
+    events = []
+    dev = [torch.from_numpy(x).cuda() for x in (src, dst, time, feat)]
+    for lo, hi in zip(cuts[:-1], cuts[1:]):
+        g.advance(*(x[lo:hi] for x in dev))
+        events.append((src[lo:hi], dst[lo:hi], time[lo:hi], feat[lo:hi], lo))
+    g.freeze_csr()
+    ref = O.csr_freeze(N, d, events)
+    assert np.array_equal(g._offsets.cpu().numpy(), ref.offsets)
+    assert np.array_equal(g._nbr_ids.cpu().numpy(), ref.ids)
+    assert np.array_equal(g._nbr_times.cpu().numpy().view(np.int64), ref.times.view(np.int64))
+    assert np.array_equal(g._nbr_feats.cpu().numpy(), ref.feats)
+    assert np.array_equal(g._nbr_eids.cpu().numpy(), ref.eids)
+    assert g.status()["bad_event_nodes"] == 0
+    return g
+
+
+@pytest.mark.parametrize("E", [2047, 2048, 2049, 4097, 9000])
+@pytest.mark.parametrize("run", [1, 3, 2048, 5000, 100_000])
+def test_segments_across_tiles(E, run):
+    rng = np.random.default_rng(E + run)
+    src, dst = rng.integers(0, 50, E), rng.integers(0, 50, E)
+    time = 10.0 + np.floor((np.arange(E) + 7) / run)
+    cuts = sorted({0, 1, 31, 32, 2047, 2048, 2049, 4096, 6000, E} & set(range(E + 1)))
+    g = _check(50, 3, cuts, src, dst, time)
+    if run > 1:
+        assert g._csr_build_mode == "runs"
+    # the same calls with a step back inside them: the time sort over whole calls
+    time[E // 2] -= 5.0
+    assert _check(50, 3, cuts, src, dst, time)._csr_build_mode == "sort"
+
+
+@pytest.mark.parametrize("E,N,d,order", [
+    (524_287, 700, 8, "strict"), (524_288, 1 << 20, 4, "ties"), (530_000, 1023, 65, "ties"),
+    (1_048_577, 1024, 4, "ties"), (1_100_000, 3, 1, "shuffled"), (2_200_000, 300_000, 2, "strict")])
+def test_sort_and_gather_sizes(E, N, d, order):
+    rng = np.random.default_rng(E)
+    skew = rng.random(E)
+    src = np.minimum((N * skew ** 6).astype(np.int64), N - 1)  # a few nodes hold most entries
+    dst = rng.integers(0, N, E)
+    time = 5.0 + np.arange(E, dtype=np.float64)
+    if order == "ties":
+        time = np.floor(time / 3.0)
+    elif order == "shuffled":
+        time = time.reshape(-1, 100)[:, ::-1].reshape(-1).copy()
+    g = _check(N, d, [0, E // 3, E], src, dst, time)
+    assert g._csr_build_mode == {"strict": "pairs", "ties": "runs", "shuffled": "sort"}[order]

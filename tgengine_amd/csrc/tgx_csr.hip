@@ -5,11 +5,12 @@
 // stably by time and then stably by node, so a node's entries end up
 // time-ascending with ties in build order (the reference's two stable
 // argsorts, :156-158).  The same permutation comes out of a stable LSD radix
-// sort: eight 8-bit passes over an order-preserving 64-bit image of the time,
-// then ceil(log2 N / 8) passes over the node id.
+// sort: seven passes over an order-preserving 64-bit image of the time, then
+// ceil(log2 N / 10) passes over the node id.
 //
-// The passes are tgx_radix.h's.  Then offsets[u] = lower_bound(sorted nodes, u), and one gather writes the
-// ids, times, edge ids and feature rows (16-byte vectors where aligned).
+// The passes are tgx_radix.h's.  Then offsets[u] = lower_bound(sorted nodes, u), and
+// one gather writes the ids, times, edge ids and feature rows (16-byte vectors
+// where aligned).
 //
 // Event pairs (TGX_CSR_EVENT_PAIRS): the caller hands the events themselves in
 // an order whose entries 2k, 2k+1 are already the stable time order of the
@@ -19,6 +20,8 @@
 
 namespace tgx {
 namespace {
+
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 // order-preserving image of a float64: -0.0 maps to +0.0 and every NaN to one
 // NaN above +inf, so ties are exactly the ties of a float comparison
@@ -42,42 +45,6 @@ __global__ __launch_bounds__(kThreads) void csr_init(const double* __restrict__ 
   idx[j] = static_cast<uint32_t>(j);
 }
 
-// entry j of the input: its node, neighbour, time index and event index
-// (pairs: entry 2k = from[k] -> to[k], 2k + 1 = to[k] -> from[k], of event k)
-struct Entries {
-  const int64_t* from;
-  const int64_t* to;
-  const int64_t* event;
-  int pairs;
-  __device__ __forceinline__ int64_t node(int64_t j) const {
-    return pairs ? ((j & 1) ? to[j >> 1] : from[j >> 1]) : from[j];
-  }
-  __device__ __forceinline__ int64_t nbr(int64_t j) const {
-    return pairs ? ((j & 1) ? from[j >> 1] : to[j >> 1]) : to[j];
-  }
-  __device__ __forceinline__ int64_t row(int64_t j) const { return pairs ? j >> 1 : j; }
-  __device__ __forceinline__ int64_t ev(int64_t j) const {
-    return event != nullptr ? event[row(j)] : (pairs ? j >> 1 : -1);
-  }
-};
-
-__global__ __launch_bounds__(kThreads) void csr_node_keys(Entries E,
-                                                          const uint32_t* __restrict__ idx,
-                                                          int64_t n, int64_t N,
-                                                          uint32_t* __restrict__ nkey,
-                                                          int32_t* __restrict__ status) {
-  const int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  bool bad = false;
-  if (p < n) {
-    const int64_t u = E.node(idx != nullptr ? idx[p] : p);  // NULL: the identity
-    bad = u < 0 || u >= N;
-    nkey[p] = bad ? 0xffffffffu : static_cast<uint32_t>(u);
-  }
-  const uint64_t bm = __ballot(bad);
-  if ((threadIdx.x & (kWave - 1)) == 0 && bm != 0 && status != nullptr)
-    atomicAdd(&status[TGX_ST_BAD_EVENT_NODE], __popcll(bm));
-}
-
 // offsets[u] = #sorted node keys < u, u in [0, N]
 __global__ __launch_bounds__(kThreads) void csr_offsets(const uint32_t* __restrict__ nkey, int64_t n,
                                                         int64_t N, int64_t* __restrict__ offsets) {
@@ -92,41 +59,6 @@ __global__ __launch_bounds__(kThreads) void csr_offsets(const uint32_t* __restri
       hi = mid;
   }
   offsets[u] = lo;
-}
-
-// out[p] = entry perm[p]: id, time, edge id, feature row (tpe lanes per row)
-template <int VEC>
-__global__ __launch_bounds__(kThreads) void csr_gather(
-    const uint32_t* __restrict__ perm, int64_t n, Entries E,
-    const double* __restrict__ time, int64_t num_events,
-    const uint8_t* __restrict__ feats, int64_t row_bytes, int tpe_log2,
-    int32_t* __restrict__ out_ids, double* __restrict__ out_times, int64_t* __restrict__ out_eids,
-    uint8_t* __restrict__ out_feats, int32_t* __restrict__ status) {
-  using V = typename std::conditional<VEC == 16, uint4, typename std::conditional<VEC == 4, uint32_t, uint16_t>::type>::type;
-  const int tpe = 1 << tpe_log2;
-  const int64_t p = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) >> tpe_log2;
-  const int l = threadIdx.x & (tpe - 1);
-  bool bad = false;
-  if (p < n) {
-    const int64_t j = perm[p];
-    const int64_t ev = E.ev(j);
-    if (l == 0) {
-      out_ids[p] = static_cast<int32_t>(E.nbr(j));
-      out_times[p] = time[E.row(j)];
-      if (out_eids != nullptr) out_eids[p] = ev;
-    }
-    if (out_feats != nullptr && row_bytes > 0) {
-      const int nv = static_cast<int>(row_bytes / VEC);
-      V* drow = reinterpret_cast<V*>(out_feats + p * row_bytes);
-      const bool have = feats != nullptr && ev >= 0 && ev < num_events;
-      bad = feats != nullptr && !have;
-      const V* srow = have ? reinterpret_cast<const V*>(feats + ev * row_bytes) : nullptr;
-      for (int c = l; c < nv; c += tpe) drow[c] = have ? srow[c] : V{};
-    }
-  }
-  const uint64_t bm = __ballot(bad && l == 0);
-  if ((threadIdx.x & (kWave - 1)) == 0 && bm != 0 && status != nullptr)
-    atomicAdd(&status[TGX_ST_BAD_EVENT_NODE], __popcll(bm));
 }
 
 // Pre-freeze scan (tgx_csr_scan): node range, time order and largest time of the
@@ -224,56 +156,298 @@ __global__ __launch_bounds__(kThreads) void csr_scan_final(const ScanPart* __res
 // segments: the advance() calls, or with TGX_CSR_NONDECREASING the runs of equal
 // times within a call.  The entries of segment [s, e) take build-order positions
 // [2s, 2e) -- from->to of event k at s + k, then to->from at e + k -- which for
-// runs of a non-decreasing stream is already its stable time order.  The
-// segment of event k comes from an exclusive scan of the segment-start marks,
-// so any call starts give a permutation of [0, 2E).
-__global__ __launch_bounds__(kThreads) void csr_seg_marks(const double* __restrict__ time, int64_t E, int runs,
-                                                          uint32_t* __restrict__ mark, uint32_t* __restrict__ ex) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (k >= E) return;
-  const uint32_t f = k == 0 || (runs && !(time[k] == time[k - 1]));
-  mark[k] = f;
-  ex[k] = f;
+// runs of a non-decreasing stream is already its stable time order.
+//
+// Two launches over tiles of kSegTile events.  Both mark the tile's segment
+// starts in an LDS bitmap (the same marks from the same inputs, so the segments
+// partition the events whatever the call starts hold): csr_seg_tiles writes each
+// tile's first and last start; csr_seg_order finds the starts nearest to its tile
+// from those, then each event's own segment from the bitmap, and writes the
+// entries at their positions.  8M events in runs of three take 13 + 91 us, the keys
+// and records of the next steps included (448 MB; before, marks, a device-wide scan
+// of them, segment starts, the order and the node keys took eight launches and 230 us).
+constexpr int kSegItems = 8;
+constexpr int kSegTile = kThreads * kSegItems;
+constexpr int kSegWords = kSegTile / 32;
+static_assert(kSegWords == kWave, "one bitmap word per lane");
+constexpr uint32_t kNoStart = 0xffffffffu;
+
+// bits[] = segment starts of events [base, base + kSegTile) (workgroup-wide; ends
+// with a barrier)
+__device__ __forceinline__ void seg_marks(const double* __restrict__ time, int64_t E, int runs,
+                                          const int64_t* __restrict__ starts, int64_t m, int64_t base,
+                                          uint32_t* bits) {
+  if (threadIdx.x < kSegWords) bits[threadIdx.x] = 0u;
+  // first call start at or after base, by 64-ary rounds of every wave
+  const int lane = threadIdx.x & (kWave - 1);
+  int64_t lo = 0, hi = m;
+  while (hi > lo) {  // wave-uniform
+    const int64_t step = (hi - lo + kWave - 1) / kWave;
+    const int64_t pos = lo + static_cast<int64_t>(lane + 1) * step - 1;
+    const int c = __popcll(__ballot(pos < hi && starts[pos] < base));
+    const int64_t nl = lo + c * step;
+    const int64_t nh = lo + (c + 1) * step - 1;
+    lo = nl < hi ? nl : hi;
+    hi = nh < hi ? nh : hi;
+  }
+  __syncthreads();
+  const int64_t end = base + kSegTile < E ? base + kSegTile : E;
+  for (int64_t c = lo + threadIdx.x; c < m; c += kThreads) {
+    const int64_t k = starts[c];
+    if (k >= end) break;
+    if (k >= 1 && k >= base) atomicOr(&bits[(k - base) >> 5], 1u << ((k - base) & 31));
+  }
+#pragma unroll
+  for (int r = 0; r < kSegItems; ++r) {
+    const int i = r * kThreads + static_cast<int>(threadIdx.x);
+    const int64_t k = base + i;
+    const bool f = k < E && (k == 0 || (runs && !(time[k] == time[k - 1])));
+    const uint64_t b = __ballot(f);
+    if ((lane & 31) == 0) {
+      const uint32_t w = lane == 0 ? static_cast<uint32_t>(b) : static_cast<uint32_t>(b >> 32);
+      if (w != 0) atomicOr(&bits[i >> 5], w);
+    }
+  }
+  __syncthreads();
 }
 
-__global__ __launch_bounds__(kThreads) void csr_seg_calls(const int64_t* __restrict__ starts, int64_t m, int64_t E,
-                                                          uint32_t* __restrict__ mark, uint32_t* __restrict__ ex) {
-  const int64_t c = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (c >= m) return;
-  const int64_t k = starts[c];
-  if (k >= 1 && k < E) {
-    mark[k] = 1;
-    ex[k] = 1;
+// first[tile], last[tile]: the tile's first and last segment start (kNoStart: none)
+__global__ __launch_bounds__(kThreads) void csr_seg_tiles(const double* __restrict__ time, int64_t E, int runs,
+                                                          const int64_t* __restrict__ starts, int64_t m,
+                                                          uint32_t* __restrict__ first, uint32_t* __restrict__ last) {
+  __shared__ uint32_t bits[kSegWords];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kSegTile;
+  seg_marks(time, E, runs, starts, m, base, bits);
+  if (threadIdx.x < kWave) {
+    const uint32_t w = bits[threadIdx.x];
+    const uint64_t any = __ballot(w != 0);
+    if (any == 0) {
+      if (threadIdx.x == 0) first[blockIdx.x] = last[blockIdx.x] = kNoStart;
+    } else {
+      const uint32_t at = static_cast<uint32_t>(base) + threadIdx.x * 32;
+      if (static_cast<int>(threadIdx.x) == __builtin_ctzll(any)) first[blockIdx.x] = at + __builtin_ctz(w);
+      if (static_cast<int>(threadIdx.x) == 63 - __builtin_clzll(any)) last[blockIdx.x] = at + 31 - __builtin_clz(w);
+    }
   }
 }
 
-// gs[segment] = its first event, gs[number of segments] = E
-__global__ __launch_bounds__(kThreads) void csr_seg_starts(const uint32_t* __restrict__ mark,
-                                                           const uint32_t* __restrict__ ex, int64_t E,
-                                                           uint32_t* __restrict__ gs) {
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (k >= E) return;
-  if (mark[k]) gs[ex[k]] = static_cast<uint32_t>(k);
-  if (k == E - 1) gs[ex[k] + mark[k]] = static_cast<uint32_t>(E);
+// the value nearest to tile `t` in direction `dir` (-1, 1) among v[0, nt) that is
+// not kNoStart, else `none`; one wavefront
+__device__ __forceinline__ uint32_t nearest_start(const uint32_t* __restrict__ v, int64_t t, int64_t nt, int dir,
+                                                  uint32_t none) {
+  const int lane = threadIdx.x & (kWave - 1);
+  for (int64_t i = t + dir; i >= 0 && i < nt; i += dir * kWave) {  // wave-uniform
+    const int64_t j = i + static_cast<int64_t>(dir) * lane;
+    const uint32_t x = j >= 0 && j < nt ? v[j] : kNoStart;
+    const uint64_t any = __ballot(x != kNoStart);
+    if (any != 0) return static_cast<uint32_t>(__shfl(static_cast<int>(x), __builtin_ctzll(any)));
+  }
+  return none;
 }
 
-// idx[position] = entry (2k + direction); tkey (when the time passes follow) its time key
-__global__ __launch_bounds__(kThreads) void csr_seg_order(const uint32_t* __restrict__ mark,
-                                                          const uint32_t* __restrict__ ex,
-                                                          const uint32_t* __restrict__ gs,
-                                                          const double* __restrict__ time, int64_t E,
-                                                          uint32_t* __restrict__ idx, uint64_t* __restrict__ tkey) {
+// event record of the row gather: time and both ends
+struct alignas(16) EventRec {
+  double time;
+  int32_t from, to;
+};
+
+// key of node u, out-of-range ones last
+__device__ __forceinline__ uint32_t node_key(int64_t u, int64_t N) {
+  return u < 0 || u >= N ? 0xffffffffu : static_cast<uint32_t>(u);
+}
+
+// idx[position] = entry (2k + direction); with RUNS also its node key and the
+// event's record, without its time key (the time passes follow)
+template <bool RUNS>
+__global__ __launch_bounds__(kThreads) void csr_seg_order(
+    const double* __restrict__ time, const int64_t* __restrict__ from, const int64_t* __restrict__ to, int64_t E,
+    int64_t N, const int64_t* __restrict__ starts, int64_t m, const uint32_t* __restrict__ first,
+    const uint32_t* __restrict__ last, uint32_t* __restrict__ idx, uint64_t* __restrict__ tkey,
+    uint32_t* __restrict__ nkey, EventRec* __restrict__ rec, int32_t* __restrict__ status) {
+  __shared__ uint32_t bits[kSegWords], prev[kSegWords], next[kSegWords], edge[2];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kSegTile;
+  // the starts around the tile: event 0 is always one, the end of the last segment is E
+  if (threadIdx.x < kWave) {
+    const uint32_t x = nearest_start(last, blockIdx.x, gridDim.x, -1, 0u);
+    if (threadIdx.x == 0) edge[0] = x;
+  } else if (threadIdx.x < 2 * kWave) {
+    const uint32_t x = nearest_start(first, blockIdx.x, gridDim.x, 1, static_cast<uint32_t>(E));
+    if (threadIdx.x == kWave) edge[1] = x;
+  }
+  seg_marks(time, E, RUNS ? 1 : 0, starts, m, base, bits);
+  if (threadIdx.x < kWave) {
+    // the last start before word `lane` and the first one after it
+    const int lane = threadIdx.x;
+    const uint32_t w = bits[lane];
+    const uint32_t at = static_cast<uint32_t>(base) + lane * 32;
+    const uint64_t any = __ballot(w != 0);
+    const uint32_t wl = w != 0 ? at + 31 - __builtin_clz(w) : 0u;
+    const uint32_t wf = w != 0 ? at + __builtin_ctz(w) : 0u;
+    const uint64_t lower = any & ((uint64_t(1) << lane) - 1);
+    const uint64_t upper = lane == 63 ? 0 : any >> (lane + 1);
+    const uint32_t pl = __shfl(wl, lower != 0 ? 63 - __builtin_clzll(lower) : 0);
+    const uint32_t nf = __shfl(wf, upper != 0 ? lane + 1 + __builtin_ctzll(upper) : 0);
+    prev[lane] = lower != 0 ? pl : edge[0];
+    next[lane] = upper != 0 ? nf : edge[1];
+  }
+  __syncthreads();
+  int bad = 0;
+#pragma unroll
+  for (int r = 0; r < kSegItems; ++r) {
+    const int i = r * kThreads + static_cast<int>(threadIdx.x);
+    const int64_t k = base + i;
+    if (k < E) {
+      const uint32_t w = bits[i >> 5];
+      const uint32_t upto = (2u << (i & 31)) - 1u;  // bits of the word up to event k
+      const uint32_t at = static_cast<uint32_t>(base) + (i & ~31);
+      const uint32_t s = (w & upto) != 0 ? at + 31 - __builtin_clz(w & upto) : prev[i >> 5];
+      const uint32_t e = (w & ~upto) != 0 ? at + __builtin_ctz(w & ~upto) : next[i >> 5];
+      const int64_t pf = static_cast<int64_t>(s) + k;
+      const int64_t pr = static_cast<int64_t>(e) + k;
+      idx[pf] = static_cast<uint32_t>(2 * k);
+      idx[pr] = static_cast<uint32_t>(2 * k + 1);
+      if constexpr (RUNS) {
+        const int64_t u = from[k], v = to[k];
+        nkey[pf] = node_key(u, N);
+        nkey[pr] = node_key(v, N);
+        bad += (u < 0 || u >= N) + (v < 0 || v >= N);
+        rec[k] = EventRec{time[k], static_cast<int32_t>(u), static_cast<int32_t>(v)};
+      } else {
+        const uint64_t key = time_key(time[k]);
+        tkey[pf] = key;
+        tkey[pr] = key;
+      }
+    }
+  }
+  if (RUNS && bad != 0 && status != nullptr) atomicAdd(&status[TGX_ST_BAD_EVENT_NODE], bad);
+}
+
+// Node keys of the event-pair build (entry 2k = from[k] -> to[k], 2k + 1 = to[k] ->
+// from[k], already in stable time order) and the events' records.
+__global__ __launch_bounds__(kThreads) void csr_pair_keys(const double* __restrict__ time,
+                                                          const int64_t* __restrict__ from,
+                                                          const int64_t* __restrict__ to, int64_t E, int64_t N,
+                                                          uint32_t* __restrict__ nkey, EventRec* __restrict__ rec,
+                                                          int32_t* __restrict__ status) {
   const int64_t k = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (k >= E) return;
-  const uint32_t g = ex[k] + mark[k] - 1;
-  const int64_t pf = static_cast<int64_t>(gs[g]) + k;
-  const int64_t pr = static_cast<int64_t>(gs[g + 1]) + k;
-  idx[pf] = static_cast<uint32_t>(2 * k);
-  idx[pr] = static_cast<uint32_t>(2 * k + 1);
-  if (tkey != nullptr) {
-    const uint64_t key = time_key(time[k]);
-    tkey[pf] = key;
-    tkey[pr] = key;
+  int bad = 0;
+  if (k < E) {
+    const int64_t u = from[k], v = to[k];
+    reinterpret_cast<uint2*>(nkey)[k] = make_uint2(node_key(u, N), node_key(v, N));
+    bad = (u < 0 || u >= N) + (v < 0 || v >= N);
+    rec[k] = EventRec{time[k], static_cast<int32_t>(u), static_cast<int32_t>(v)};
+  }
+  if (bad != 0 && status != nullptr) atomicAdd(&status[TGX_ST_BAD_EVENT_NODE], bad);
+}
+
+// records of events (or, where entries are given one by one, of entries)
+__global__ __launch_bounds__(kThreads) void csr_records(const double* __restrict__ time,
+                                                        const int64_t* __restrict__ from,
+                                                        const int64_t* __restrict__ to, int64_t E,
+                                                        EventRec* __restrict__ rec) {
+  const int64_t k = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (k < E) rec[k] = EventRec{time[k], static_cast<int32_t>(from[k]), static_cast<int32_t>(to[k])};
+}
+
+// nkey[p] = node of entry idx[p] (pairs: entry 2k is from[k]'s, 2k + 1 to[k]'s)
+__global__ __launch_bounds__(kThreads) void csr_node_keys(const int64_t* __restrict__ from,
+                                                          const int64_t* __restrict__ to, int pairs,
+                                                          const uint32_t* __restrict__ idx, int64_t n, int64_t N,
+                                                          uint32_t* __restrict__ nkey, int32_t* __restrict__ status) {
+  const int64_t p = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  bool bad = false;
+  if (p < n) {
+    const uint32_t j = idx[p];
+    const int64_t u = pairs ? ((j & 1) ? to[j >> 1] : from[j >> 1]) : from[j];
+    bad = u < 0 || u >= N;
+    nkey[p] = node_key(u, N);
+  }
+  const uint64_t bm = __ballot(bad);
+  if ((threadIdx.x & (kWave - 1)) == 0 && bm != 0 && status != nullptr)
+    atomicAdd(&status[TGX_ST_BAD_EVENT_NODE], __popcll(bm));
+}
+
+// out[p] = entry perm[p]: id, time, edge id, feature row.  The entries of a node
+// come from all over the stream, and every read of a 16-byte record (neighbour and
+// time: before, two 8-byte reads from two arrays) or a short row fetches a 128-byte
+// line: node by node, 16M entries with 32-byte rows fetched 2.9 GB for 0.8 GB used,
+// in 548 us (674 with the two arrays).  So tiles of `per` consecutive entries run
+// in the order of their first events: the busy nodes, which hold most of a skewed
+// stream's entries, then walk the stream together and share its lines, and runs of
+// kGatherSlice such tiles go to one XCD, for its L2: 353 us, and 23 us for the order.
+// A workgroup takes one tile, its permutation in LDS, and copies the rows as one
+// run of chunks, kGatherDepth per thread loaded before the first is stored,
+// whatever the row's width (314,948 entries with 688-byte rows: 118 -> 75 us
+// against a row per wavefront).  Output leaves as nontemporal stores, which leaves
+// the caches to the events (5 of 80 us on those).
+constexpr int kGatherDepth = 4;
+constexpr int kGatherChunks = kThreads * kGatherDepth;  // chunks a workgroup holds in flight
+constexpr int kGatherMost = 512;                        // entries per workgroup at most
+constexpr int kXcds = 8;
+constexpr int kGatherSlice = 64;  // tiles of neighbouring events given to one XCD
+
+// key of tile i (`per` entries) of the gather: its first entry's event
+__global__ __launch_bounds__(kThreads) void csr_tile_keys(const uint32_t* __restrict__ perm, int64_t ntiles, int per,
+                                                          int pairs, uint32_t* __restrict__ key) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  if (i < ntiles) key[i] = perm[i * per] >> (pairs ? 1 : 0);
+}
+
+template <int VEC>
+__global__ __launch_bounds__(kThreads) void csr_gather(
+    const uint32_t* __restrict__ perm, int64_t n, const EventRec* __restrict__ rec, int pairs,
+    const int64_t* __restrict__ event, int64_t num_events, const uint8_t* __restrict__ feats, int nch,
+    uint32_t nch_magic, int per, const uint32_t* __restrict__ order, int64_t ntiles, int32_t* __restrict__ out_ids, double* __restrict__ out_times,
+    int64_t* __restrict__ out_eids, uint8_t* __restrict__ out_feats, int32_t* __restrict__ status) {
+  using V = typename std::conditional<VEC == 16, u32x4,
+                                      typename std::conditional<VEC == 4, uint32_t, uint16_t>::type>::type;
+  __shared__ int64_t row[kGatherMost];  // an entry's feature row, -1: zeros
+  int64_t tile = blockIdx.x;
+  if (order != nullptr) {  // launch-uniform
+    const int64_t g = tile / (kXcds * kGatherSlice);
+    const int r = static_cast<int>(tile - g * (kXcds * kGatherSlice));
+    const int64_t at = (g * kXcds + r % kXcds) * kGatherSlice + r / kXcds;
+    if (at >= ntiles) return;  // workgroup-uniform
+    tile = order[at];
+  }
+  const int64_t p0 = tile * per;
+  const int cnt = static_cast<int>(n - p0 < per ? n - p0 : per);
+  for (int i = threadIdx.x; i < cnt; i += kThreads) {
+    const uint32_t j = perm[p0 + i];
+    const int64_t k = pairs ? j >> 1 : j;
+    const EventRec r = rec[k];
+    const int64_t ev = event != nullptr ? event[k] : (pairs ? k : -1);
+    const bool have = feats != nullptr && ev >= 0 && ev < num_events;
+    row[i] = have ? ev : -1;
+    __builtin_nontemporal_store(pairs && (j & 1) ? r.from : r.to, out_ids + p0 + i);
+    __builtin_nontemporal_store(r.time, out_times + p0 + i);
+    if (out_eids != nullptr) out_eids[p0 + i] = ev;
+    if (out_feats != nullptr && feats != nullptr && !have && status != nullptr)
+      atomicAdd(&status[TGX_ST_BAD_EVENT_NODE], 1);
+  }
+  if (out_feats == nullptr) return;  // launch-uniform
+  __syncthreads();
+  const V* src = reinterpret_cast<const V*>(feats);
+  V* dst = reinterpret_cast<V*>(out_feats) + p0 * nch;
+  const int64_t total = static_cast<int64_t>(cnt) * nch;
+  for (int64_t c0 = threadIdx.x; c0 < total; c0 += kGatherChunks) {
+    V v[kGatherDepth];
+#pragma unroll
+    for (int u = 0; u < kGatherDepth; ++u) {
+      const int64_t c = c0 + u * kThreads;
+      v[u] = V{};
+      if (c < total) {
+        // one entry per workgroup, or a dividend below 2^32 / nch
+        const int e = per == 1 ? 0 : nch == 1 ? static_cast<int>(c) : static_cast<int>(__umulhi(static_cast<uint32_t>(c), nch_magic));
+        const int64_t ev = row[e];
+        if (ev >= 0) v[u] = src[ev * nch + (c - static_cast<int64_t>(e) * nch)];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kGatherDepth; ++u) {
+      const int64_t c = c0 + u * kThreads;
+      if (c < total) __builtin_nontemporal_store(v[u], dst + c);
+    }
   }
 }
 
@@ -291,7 +465,7 @@ Layout layout(int64_t n) {
   w.nkey = w.idx + 2 * align256(un * 4);
   w.count = w.nkey + 2 * align256(un * 4);
   w.sums = w.count + w.r.count_bytes;
-  w.total = w.sums + w.r.sums_bytes;
+  w.total = w.sums + w.r.sums_bytes + 16;  // the sections start at a multiple of 16
   return w;
 }
 
@@ -347,7 +521,7 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
   if (a->workspace == nullptr || a->workspace_bytes < w.total)
     return fail(TGX_ERR_ARG, "tgx_csr_build: workspace of %zu bytes needed, got %zu", w.total,
                 a->workspace_bytes);
-  uint8_t* ws = static_cast<uint8_t*>(a->workspace);
+  uint8_t* ws = reinterpret_cast<uint8_t*>((reinterpret_cast<uintptr_t>(a->workspace) + 15) & ~uintptr_t(15));
   const unsigned g1 = static_cast<unsigned>(std::max<int64_t>(cdiv(n, kThreads), 1));
   int rc;
   if (n == 0) {
@@ -364,48 +538,52 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
                      reinterpret_cast<uint32_t*>(ws + w.nkey + align256(un * 4))};
   uint32_t* count = reinterpret_cast<uint32_t*>(ws + w.count);
   uint32_t* sums = reinterpret_cast<uint32_t*>(ws + w.sums);
-  const Entries E{a->from, a->to, a->event, pairs};
+  // the row gather's records take the time keys' place, once those are sorted
+  EventRec* rec = reinterpret_cast<EventRec*>(ws + w.tkey);
+  const int64_t ne = pairs ? n / 2 : n;  // events, or entries given one by one
+  const unsigned ge = static_cast<unsigned>(cdiv(ne, kThreads));
   int cur = 0;
+  const bool ident = pairs && !by_call;  // already in stable time order
+  bool keyed = false;                    // node keys and records are done
   if (by_call) {
-    // the build order from the segments; marks and their scan in nk[0], the
-    // segment starts in nk[1], the scan's tile sums in the digit counts (free
-    // until the first pass)
-    const int64_t ne = n / 2;
-    const unsigned ge = static_cast<unsigned>(cdiv(ne, kThreads));
-    uint32_t* mark = nk[0];
-    uint32_t* ex = nk[0] + ne;
-    hipLaunchKernelGGL(csr_seg_marks, dim3(ge), dim3(kThreads), 0, stream, a->time, ne, runs, mark, ex);
-    if ((rc = check_launch("csr_seg_marks"))) return rc;
-    if (a->num_calls > 0) {
-      hipLaunchKernelGGL(csr_seg_calls, dim3(static_cast<unsigned>(cdiv(a->num_calls, kThreads))), dim3(kThreads), 0,
-                         stream, a->call_starts, a->num_calls, ne, mark, ex);
-      if ((rc = check_launch("csr_seg_calls"))) return rc;
-    }
-    if ((rc = scan_exclusive(ex, ne, count, scan_levels(ne), 0, stream))) return rc;
-    hipLaunchKernelGGL(csr_seg_starts, dim3(ge), dim3(kThreads), 0, stream, static_cast<const uint32_t*>(mark),
-                       static_cast<const uint32_t*>(ex), ne, nk[1]);
-    if ((rc = check_launch("csr_seg_starts"))) return rc;
-    hipLaunchKernelGGL(csr_seg_order, dim3(ge), dim3(kThreads), 0, stream, static_cast<const uint32_t*>(mark),
-                       static_cast<const uint32_t*>(ex), static_cast<const uint32_t*>(nk[1]), a->time, ne, ix[0],
-                       runs ? static_cast<uint64_t*>(nullptr) : tk[0]);
+    // the build order from the segments; each tile's starts in nk[1] (free until the first pass)
+    const unsigned gt = static_cast<unsigned>(cdiv(ne, kSegTile));
+    uint32_t* first = nk[1];
+    uint32_t* last = nk[1] + gt;
+    hipLaunchKernelGGL(csr_seg_tiles, dim3(gt), dim3(kThreads), 0, stream, a->time, ne, runs, a->call_starts,
+                       a->num_calls, first, last);
+    if ((rc = check_launch("csr_seg_tiles"))) return rc;
+    auto order = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(gt), dim3(kThreads), 0, stream, a->time, a->from, a->to, ne, N, a->call_starts,
+                         a->num_calls, static_cast<const uint32_t*>(first), static_cast<const uint32_t*>(last), ix[0],
+                         tk[0], nk[0], rec, a->status);
+    };
+    if (runs)
+      order(csr_seg_order<true>);
+    else
+      order(csr_seg_order<false>);
     if ((rc = check_launch("csr_seg_order"))) return rc;
+    keyed = runs != 0;
     // stable by time unless the runs already are
     if (!runs && (rc = radix_sort<uint64_t>(tk, ix, cur, n, 64, w.r, count, sums, stream))) return rc;
-  } else if (pairs) {
-    // already in stable time order: the identity, which the node keys and the
-    // first node pass take without reading it
+  } else if (ident) {
+    hipLaunchKernelGGL(csr_pair_keys, dim3(ge), dim3(kThreads), 0, stream, a->time, a->from, a->to, ne, N, nk[0], rec,
+                       a->status);
+    if ((rc = check_launch("csr_pair_keys"))) return rc;
+    keyed = true;
   } else {
     hipLaunchKernelGGL(csr_init, dim3(g1), dim3(kThreads), 0, stream, a->time, n, tk[0], ix[0]);
     if ((rc = check_launch("csr_init"))) return rc;
-    // stable by time: 8 passes, ping-pong ending in buffer 0
     if ((rc = radix_sort<uint64_t>(tk, ix, cur, n, 64, w.r, count, sums, stream))) return rc;
   }
   // then stable by node over ceil(log2 N) bits (out-of-range ids sort last)
-  const bool ident = pairs && !by_call;
-  hipLaunchKernelGGL(csr_node_keys, dim3(g1), dim3(kThreads), 0, stream, E,
-                     ident ? static_cast<const uint32_t*>(nullptr) : static_cast<const uint32_t*>(ix[cur]), n, N,
-                     nk[0], a->status);
-  if ((rc = check_launch("csr_node_keys"))) return rc;
+  if (!keyed) {
+    hipLaunchKernelGGL(csr_records, dim3(ge), dim3(kThreads), 0, stream, a->time, a->from, a->to, ne, rec);
+    if ((rc = check_launch("csr_records"))) return rc;
+    hipLaunchKernelGGL(csr_node_keys, dim3(g1), dim3(kThreads), 0, stream, a->from, a->to, pairs,
+                       static_cast<const uint32_t*>(ix[cur]), n, N, nk[0], a->status);
+    if ((rc = check_launch("csr_node_keys"))) return rc;
+  }
   int bits = 1;
   while ((int64_t(1) << bits) < N + 1) ++bits;  // + 1: the out-of-range key 0xffffffff
   // the node keys ride in nk[], the permutation in ix[] (starting where the time
@@ -424,15 +602,35 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
     vec = 16;
   else if (row_bytes % 4 == 0 && (!fe || (al(a->feats, 3) && al(a->out_feats, 3))))
     vec = 4;
-  const int64_t nchunks = fe ? row_bytes / vec : 1;
-  int tpe_log2 = 0;
-  while ((int64_t(1) << tpe_log2) < nchunks && tpe_log2 < 6) ++tpe_log2;
-  const dim3 gg(static_cast<unsigned>(cdiv(n << tpe_log2, kThreads)));
+  const int64_t nch = fe ? row_bytes / vec : 1;
+  const int per = static_cast<int>(std::min<int64_t>(std::max<int64_t>(kGatherChunks / nch, 1), kGatherMost));
+  const uint32_t magic = nch > 1 ? 0xffffffffu / static_cast<uint32_t>(nch) + 1u : 0u;
+  const int64_t ntiles = cdiv(n, per);
+  int64_t gblocks = ntiles;
+  const uint32_t* order = nullptr;
+  // Rows of at most 256 bytes and at least 1M entries: below that the events fit
+  // the caches in any order, and a wider row fills its lines by itself
+  if (per >= 64 && n >= (int64_t(1) << 20)) {
+    // the node keys are done with (the offsets are out): tile keys, sorted keys and order take their place
+    uint32_t* key = nk[0];
+    uint32_t* val = nk[0] + 2 * ntiles;
+    hipLaunchKernelGGL(csr_tile_keys, dim3(static_cast<unsigned>(cdiv(ntiles, kThreads))), dim3(kThreads), 0, stream,
+                       static_cast<const uint32_t*>(perm_in), ntiles, per, pairs, key);
+    if ((rc = check_launch("csr_tile_keys"))) return rc;
+    int ebits = 1;
+    while ((int64_t(1) << ebits) < ne) ++ebits;
+    const int dbits = std::min(ebits, kMaxDigitBits);
+    if ((rc = radix_pass<uint32_t>(key, nullptr, key + ntiles, val, ntiles, ebits - dbits, dbits, radix_scratch(ntiles),
+                                   count, sums, stream)))
+      return rc;
+    order = val;
+    gblocks = cdiv(ntiles, kXcds * kGatherSlice) * (kXcds * kGatherSlice);
+  }
   auto gather = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, gg, dim3(kThreads), 0, stream, static_cast<const uint32_t*>(perm_in), n,
-                       E, a->time, a->num_events,
-                       static_cast<const uint8_t*>(a->feats), fe ? row_bytes : 0, tpe_log2, a->out_ids,
-                       a->out_times, a->out_eids, static_cast<uint8_t*>(fe ? a->out_feats : nullptr),
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(gblocks)), dim3(kThreads), 0, stream,
+                       static_cast<const uint32_t*>(perm_in), n, static_cast<const EventRec*>(rec), pairs, a->event,
+                       a->num_events, static_cast<const uint8_t*>(a->feats), static_cast<int>(nch), magic, per, order, ntiles,
+                       a->out_ids, a->out_times, a->out_eids, static_cast<uint8_t*>(fe ? a->out_feats : nullptr),
                        a->status);
   };
   if (vec == 16)

@@ -573,7 +573,7 @@ NpLayout np_layout(int64_t n) {
   w.cval = w.ckey + 2 * align256(un * 8);
   w.count = w.cval + 2 * align256(un * 4);
   w.sums = w.count + w.r.count_bytes;
-  w.total = w.sums + w.r.sums_bytes;
+  w.total = w.sums + w.r.sums_bytes + 16;  // the sort path's sections start at a multiple of 16
   return w;
 }
 
@@ -674,7 +674,7 @@ int negpool_update(const char* who, int32_t* pool, int64_t* count, int64_t num_n
                          call, status);
     return check_launch("np_update_small");
   }
-  uint8_t* ws = static_cast<uint8_t*>(workspace);
+  uint8_t* ws = reinterpret_cast<uint8_t*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~uintptr_t(15));
   const size_t un = static_cast<size_t>(n);
   uint32_t* key[2] = {reinterpret_cast<uint32_t*>(ws + w.key), reinterpret_cast<uint32_t*>(ws + w.key + align256(un * 4))};
   uint32_t* idx[2] = {reinterpret_cast<uint32_t*>(ws + w.idx), reinterpret_cast<uint32_t*>(ws + w.idx + align256(un * 4))};
