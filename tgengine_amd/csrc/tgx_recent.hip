@@ -517,15 +517,17 @@ __device__ __forceinline__ void co_occurrence_pair(const Params& P, int64_t g, i
 // gfx9 counts vector loads and stores in one in-order vmcnt, so a load behind
 // stores would wait for their completion.  With at most one wave per SIMD slot
 // for the whole grid the gathers all run up front and the stores then stream.
-// Waves-per-SIMD target: 8 for the event- and list-plan kernels with rows through
-// memory, whose bandwidth needs every resident wave (plan-group workgroups of 6
-// waves fit 5 per CU at 8, 4 at 7; without the target C5's gather took 200 us
-// instead of 176); none for the small-row kernels and the tiled 16-byte-chunk
-// kernel, where forcing 8 capped the scalar registers and spilled them into their
-// own code (the tiled one: 8.56 -> 7.74 us on C1 and 367 -> 356 us on C4 without
-// it), while the 7 the registers allow still hold their grids.
+// Waves-per-SIMD target: 8 for the ring-only event- and list-plan kernels with rows
+// through memory, whose bandwidth needs every resident wave (plan-group workgroups
+// of 6 waves fit 5 per CU at 8, 4 at 7; without the target C5's gather took 200 us
+// instead of 176); none for the tiled kernels of 16-byte chunks and the tiled CSR
+// copies, where forcing 8 capped the scalar registers and spilled them into their
+// own code (8.56 -> 7.74 us on C1 and 367 -> 356 us on C4 without it), nor for the
+// event-plan CSR copies with rows through memory; 7 for the rest, where it keeps a
+// private segment (a scalar spill's) out of the kernel.
 template <int VEC, int NREG, bool TILES, bool CSR>
-constexpr int kWavesPerEu = CSR || NREG > 0 || (TILES && VEC == 16) ? 1 : 8;
+constexpr int kWavesPerEu = TILES ? (VEC == 16 || CSR ? 1 : 7)
+                                  : CSR ? (NREG > 0 || VEC == 2 ? 7 : 1) : (NREG > 0 ? 7 : 8);
 
 // TILES: the launch's plan mode is TGX_PLAN_TILES (no event or list plan, so no
 // co-occurrence); that copy of the kernel carries none of their code, which
@@ -968,11 +970,11 @@ void recent_fused(Params P) {
 // window then holds none), those entries are the answer, as the search would
 // find: three dependent round trips (query, offsets, entries) before the
 // stores, against five for recent_fused's search, staging and row copy.
-// Otherwise the search goes on from a first Bp-ary round whose probes went out
-// with those loads (a window of more than Bp entries and a query time not after
-// the CSR's last one: max_time), the wave searching what is left of each such
-// query's window (wave_lower_bound, as recent_fused), and the answer's entries
-// are reloaded.
+// A query that may fall inside its window (a time not after the CSR's largest one,
+// max_time, when that is finite) sends the search's first Bp-ary round in place of
+// those loads, and its entries once the search is done: loading them both ways cost
+// the entries' bytes again (12,000 queries inside their windows 13.5 -> 12.8 us; two
+// hops of 4,000 x 20, whose hop-2 queries all are, 45.3 -> 43.4 us).
 template <int NREG>
 __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
   using VT = u32x4;
@@ -1034,14 +1036,15 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
         if (k < P.nch) rows[k] = src[k];
     }
   };
-  bool have = live && sl < K && s1 - K + sl >= s0;
-  if (have) load_entry(s1 - K + sl);
-  // the search's first round over a window of more than Bp entries, when the query
-  // may be inside it (not after the CSR's last time): probe sl at s0 + (sl + 1)
-  // step - 1, clamped to the last entry
+  // A query that may be inside its window (not after the CSR's largest time, when
+  // that is known) probes instead of loading entries it would throw away: the
+  // search's first Bp-ary round, probe sl at s0 + (sl + 1) step - 1, clamped to
+  // the last entry, so the top lane reads the window's last time.
   const int Bp = 1 << lg;
   const int64_t wlen = s1 - s0;
-  const bool probing = live && wlen > Bp && qt <= P.c_tmax;
+  const bool probing = wlen > 0 && qt <= P.c_tmax && P.c_tmax < __builtin_huge_val();
+  bool have = live && sl < K && s1 - K + sl >= s0 && !probing;
+  if (have) load_entry(s1 - K + sl);
   const int64_t step = probing ? (wlen + Bp - 1) >> lg : 0;
   double tp = 0.0;
   if (probing) {
@@ -1049,11 +1052,11 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
     tp = P.c_times[pos < s1 ? pos : s1 - 1];
   }
   // sub-group uniform: lane K - 1 holds entry s1 - 1 whenever the window is not empty
-  const double tl = __shfl(t, (h << lg) + K - 1);
+  const double tl = __shfl(probing ? tp : t, (h << lg) + (probing ? Bp : K) - 1);
   const bool after = !live || s1 == s0 || tl < qt;
 
   // ---- otherwise: search the window, then load the answer's entries ----
-  const uint64_t slow = __ballot(!after);
+  const uint64_t slow = __ballot(!after || probing);
   if (slow != 0) {  // wave-uniform
     // the lower bound lies in [lo, hi]: after the first round, between the last
     // probe below the query time and the next one
@@ -1068,8 +1071,9 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
     }
     // every sub-group searches its own query at once (Bp-ary rounds; one query
     // after another with 64-ary rounds took 2 x 3 rounds for C3's hop-2 windows)
-    const int64_t cnt = subgroup_lower_bound(P.c_times, lo, hi, qt, !after, sl, h, lg) - s0;
-    if (!after) {
+    const int64_t end = subgroup_lower_bound(P.c_times, lo, hi, qt, !after, sl, h, lg);
+    if (!after || probing) {
+      const int64_t cnt = (after ? s1 : end) - s0;
       const int take = static_cast<int>(cnt < K ? cnt : K);
       have = sl < K && sl >= K - take;
       if (have) load_entry(s0 + cnt - K + sl);
@@ -1130,8 +1134,10 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
 // window's last time and the first kCopyDepth chunks per lane of its share of
 // their rows; when the query comes after its whole window those are the answer
 // (query, offsets, entries and first row chunks: three dependent round trips
-// before the first store, against five in recent_fused's ring-less copy).
-// Otherwise the wave searches the window and reloads.
+// before the first store, against five in recent_fused's ring-less copy).  A query
+// that may be inside its window searches first and then loads, as in csr_window:
+// 200 training events of a frozen Reddit-sized graph (K = 64, 688-byte rows) threw
+// away 20 MB of rows and took 17.4 us, 16.1 now.
 template <int VEC, bool RANGES>
 __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   using VT = typename Vec<VEC>::T;
@@ -1195,10 +1201,12 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
     id = P.c_ids[x];
     if (P.o_eids != nullptr) eid = P.c_eids != nullptr ? P.c_eids[x] : -1;
   };
-  bool have = live && lane < np && s1 - K + pos >= s0;
+  // A query that may be inside its window (not after the CSR's largest time, when
+  // that is known) does not load what it would throw away, but sends the search's
+  // first 64-ary round instead, clamped to the window's last entry.
+  const bool probing = s1 > s0 && qt <= P.c_tmax && P.c_tmax < __builtin_huge_val();  // wave-uniform
+  bool have = live && lane < np && s1 - K + pos >= s0 && !probing;
   if (have) load_entry(s1 - K + pos);
-  // with ranges only the last wave holds position K - 1
-  if (RANGES && live && s1 > s0) tl = P.c_times[s1 - 1];
   const bool fe = P.o_feats != nullptr && P.row_bytes > 0;
   const int nch = P.nch;
   const int total = np * nch;  // chunks of the wave's positions
@@ -1206,24 +1214,44 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   const VT* crow = reinterpret_cast<const VT*>(P.c_feats);
   VT v[kCopyDepth];
 #pragma unroll
-  for (int u = 0; u < kCopyDepth; ++u) {
-    const int idx = off + u * cstride + lane;
-    v[u] = VT{};
-    if (fe && live && idx < total) {
-      const int pl = static_cast<int>(dv.div(idx));
-      const int64_t x = s1 - K + p0 + pl;
-      if (x >= s0) v[u] = crow[x * nch + (idx - pl * nch)];
+  for (int u = 0; u < kCopyDepth; ++u) v[u] = VT{};
+  bool after = !live || s1 == s0;
+  int64_t lo = s0, hi = s1;
+  if (probing) {
+    const int64_t step = (s1 - s0 + kWave - 1) / kWave;
+    const int64_t at = s0 + (lane + 1) * step - 1;
+    const double tp = P.c_times[at < s1 ? at : s1 - 1];
+    const int c = __popcll(__ballot(tp < qt));
+    after = c == kWave;
+    const int64_t nl = s0 + c * step;
+    const int64_t pc = s0 + (c + 1) * step - 1;
+    lo = nl < s1 ? nl : s1;
+    hi = pc < s1 ? pc : s1;
+  } else {
+    // with ranges only the last wave holds position K - 1
+    if (RANGES && live && s1 > s0) tl = P.c_times[s1 - 1];
+#pragma unroll
+    for (int u = 0; u < kCopyDepth; ++u) {
+      const int idx = off + u * cstride + lane;
+      if (fe && live && idx < total) {
+        const int pl = static_cast<int>(dv.div(idx));
+        const int64_t x = s1 - K + p0 + pl;
+        if (x >= s0) v[u] = crow[x * nch + (idx - pl * nch)];
+      }
     }
+    if (!RANGES) tl = __shfl(t, K - 1);  // entry s1 - 1 whenever the window is not empty
+    after = after || tl < qt;
   }
-  if (!RANGES) tl = __shfl(t, K - 1);  // entry s1 - 1 whenever the window is not empty
-  const bool after = !live || s1 == s0 || tl < qt;
   // position p >= K - take holds entry base + p
   int64_t base = s1 - K;
   int take = live ? static_cast<int>(s1 - s0 < K ? s1 - s0 : K) : 0;
-  if (!after) {  // wave-uniform
-    const int64_t cnt = wave_lower_bound<true>(P.c_times, s0, s1, qt, lane) - s0;
-    take = static_cast<int>(cnt < K ? cnt : K);
-    base = s0 + cnt - K;
+  const bool reload = !after || probing;  // wave-uniform
+  if (reload) {
+    if (!after) {
+      const int64_t cnt = wave_lower_bound<true>(P.c_times, lo, hi, qt, lane) - s0;
+      take = static_cast<int>(cnt < K ? cnt : K);
+      base = s0 + cnt - K;
+    }
     have = lane < np && pos >= K - take;
     if (have) load_entry(base + pos);
   }
@@ -1233,7 +1261,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
     if (fe) {
       VT* of = reinterpret_cast<VT*>(P.o_feats) + (q * K + p0) * nch;
       for (int idx0 = off; idx0 < total; idx0 += kCopyDepth * cstride) {
-        if (idx0 != off || !after) {
+        if (idx0 != off || reload) {
 #pragma unroll
           for (int u = 0; u < kCopyDepth; ++u) {
             const int idx = idx0 + u * cstride + lane;
