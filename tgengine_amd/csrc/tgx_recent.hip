@@ -410,103 +410,106 @@ __device__ __forceinline__ void encode_rows(const Params& P, int64_t r0, int np,
   }
 }
 
-// Co-occurrence counts of one (query a, query c) pair by one wavefront; A and Cc
-// are the K neighbour ids of the two queries (LDS).  Output row g.
+// fn(A[j], Cc[j]) for every j < K, the ids read four at a time (both arrays start
+// at a multiple of 16 bytes)
+template <class Fn>
+__device__ __forceinline__ void for_id_pairs(const int32_t* A, const int32_t* Cc, int K, Fn&& fn) {
+  const int full = K & ~3;
+  for (int j = 0; j < full; j += 4) {
+    const int4 a = *reinterpret_cast<const int4*>(A + j);
+    const int4 c = *reinterpret_cast<const int4*>(Cc + j);
+    fn(a.x, c.x);
+    fn(a.y, c.y);
+    fn(a.z, c.z);
+    fn(a.w, c.w);
+  }
+  for (int j = full; j < K; ++j) fn(A[j], Cc[j]);
+}
+
+// Co-occurrence counts of one (query a, query c) pair by the workgroup; A and Cc
+// are the K neighbour ids of the two queries (LDS), `pairs` a zeroed LDS counter.
+// Output row g.  Every position is compared with all K of either side, so the
+// counting is K^2 work: each wavefront takes 64 positions of one side at a time
+// (one wavefront of the group did it all before: 200 pairs at K = 512 took 176 us
+// with their gather, 69.8 in this form).  At K <= 32 wave 0 takes both sides in one pass.
 __device__ __forceinline__ void co_occurrence_pair(const Params& P, int64_t g, int64_t qa, int64_t qc,
-                                                   const int32_t* A, const int32_t* Cc, int lane) {
+                                                   const int32_t* A, const int32_t* Cc, int32_t* pairs, int wv,
+                                                   int waves, int lane) {
   const int K = P.K;
-  if (P.co_mode == TGX_CO_FREQ && K <= kWave / 2) {
-    // both sides in one pass: lanes [0, 32) take A's positions, lanes [32, 64) C's
+  const bool freq = P.co_mode == TGX_CO_FREQ;
+  if (freq && K <= kWave / 2) {
+    if (wv != 0) return;
+    // lanes [0, 32) take A's positions, lanes [32, 64) C's
     const int side = lane >> 5;
     const int i = lane & 31;
     const int32_t x = i < K ? (side == 0 ? A[i] : Cc[i]) : -1;
     int na = 0, nc = 0;
-    if (x != -1) {
-      for (int j = 0; j < K; ++j) {
-        na += A[j] == x;
-        nc += Cc[j] == x;
-      }
-    }
+    for_id_pairs(A, Cc, K, [&](int32_t a, int32_t c) {
+      na += a == x;
+      nc += c == x;
+    });
+    if (x == -1) na = nc = 0;
     if (i < K) {
       int32_t* out = side == 0 ? P.co_a : P.co_c;
       out[(g * K + i) * 2 + 0] = na;
       out[(g * K + i) * 2 + 1] = nc;
     }
-    const int pc = __popcll(__ballot(side == 0 && i < K && x != -1 && nc > 0));
+    const int pc = __popcll(__ballot(side == 0 && x != -1 && nc > 0));
     if (lane == 0 && P.co_pair != nullptr) P.co_pair[g] = static_cast<float>(pc);
     return;
   }
-  if (P.co_mode == TGX_CO_FREQ) {
-    for (int side = 0; side < 2; ++side) {
-      const int32_t* X = side == 0 ? A : Cc;
-      int32_t* out = side == 0 ? P.co_a : P.co_c;
-      int pc = 0;
-      for (int i0 = 0; i0 < K; i0 += kWave) {
-        const int i = i0 + lane;
-        int32_t x = -1;
-        int na = 0, nc = 0;
-        if (i < K) {
-          x = X[i];
-          if (x != -1) {
-            for (int j = 0; j < K; ++j) {
-              na += A[j] == x;
-              nc += Cc[j] == x;
-            }
-          }
-          out[(g * K + i) * 2 + 0] = na;
-          out[(g * K + i) * 2 + 1] = nc;
-        }
-        pc += __popcll(__ballot(i < K && x != -1 && nc > 0));
-      }
-      if (side == 0 && lane == 0 && P.co_pair != nullptr) P.co_pair[g] = static_cast<float>(pc);
-    }
-    return;
-  }
   // DyGFormer counts on A' = [node_a] ++ A, C' = [node_c] ++ C (length K+1)
-  const int32_t na0 = static_cast<int32_t>(query_node(P, qa));
-  const int32_t nc0 = static_cast<int32_t>(query_node(P, qc));
-  const int L = K + 1;
-  if (P.co_pair != nullptr) {
-    // (B,) count over the K sequences, as in FREQ mode
-    int pc = 0;
-    for (int i0 = 0; i0 < K; i0 += kWave) {
-      const int i = i0 + lane;
-      bool hit = false;
-      if (i < K && A[i] != -1)
-        for (int j = 0; j < K && !hit; ++j) hit = Cc[j] == A[i];
-      pc += __popcll(__ballot(hit));
-    }
-    if (lane == 0) P.co_pair[g] = static_cast<float>(pc);
-  }
-  for (int side = 0; side < 2; ++side) {
-    int32_t* out = side == 0 ? P.co_a : P.co_c;
-    for (int i = lane; i < L; i += kWave) {
-      const int32_t ai = i == 0 ? na0 : A[i - 1];
-      const int32_t ci = i == 0 ? nc0 : Cc[i - 1];
-      int f0 = 0, f1 = 0;
+  const int32_t na0 = freq ? -1 : static_cast<int32_t>(query_node(P, qa));
+  const int32_t nc0 = freq ? -1 : static_cast<int32_t>(query_node(P, qc));
+  const int L = freq ? K : K + 1;
+  const int chunks = (L + kWave - 1) / kWave;
+  for (int w = wv; w < 2 * chunks; w += waves) {  // wave-uniform
+    const int side = w >= chunks ? 1 : 0;
+    const int i = (w - side * chunks) * kWave + lane;
+    int f0 = 0, f1 = 0;
+    if (freq) {
+      const int32_t x = i < L ? (side == 0 ? A[i] : Cc[i]) : -1;
+      for_id_pairs(A, Cc, K, [&](int32_t a, int32_t c) {
+        f0 += a == x;
+        f1 += c == x;
+      });
+      if (x == -1) f0 = f1 = 0;
+      const int pc = __popcll(__ballot(side == 0 && f1 > 0));
+      if (lane == 0 && pc > 0) atomicAdd(pairs, pc);
+    } else {
+      const int32_t ai = i >= L ? -1 : i == 0 ? na0 : A[i - 1];
+      const int32_t ci = i >= L ? -1 : i == 0 ? nc0 : Cc[i - 1];
+      int hits = 0;
       if (side == 0) {
-        if (ai != -1) {
-          for (int j = 0; j < L; ++j) {
-            const int32_t aj = j == 0 ? na0 : A[j - 1];
-            const int32_t cj = j == 0 ? nc0 : Cc[j - 1];
-            f0 += aj == ai;
-            f1 += (aj == ci) && (cj != -1);
-          }
-        }
+        f0 = na0 == ai;
+        f1 = na0 == ci && nc0 != -1;
+        for_id_pairs(A, Cc, K, [&](int32_t a, int32_t c) {
+          f0 += a == ai;
+          f1 += a == ci && c != -1;
+          hits += c == ai;
+        });
+        if (ai == -1) f0 = f1 = 0;
+        // the (B,) count covers the K sequences, as in FREQ mode
+        const int pc = __popcll(__ballot(i >= 1 && ai != -1 && hits > 0));
+        if (lane == 0 && pc > 0) atomicAdd(pairs, pc);
       } else {
-        if (ci != -1) {
-          for (int j = 0; j < L; ++j) {
-            const int32_t aj = j == 0 ? na0 : A[j - 1];
-            const int32_t cj = j == 0 ? nc0 : Cc[j - 1];
-            f0 += (cj == ai) && (aj != -1);
-            f1 += cj == ci;
-          }
-        }
+        f0 = nc0 == ai && na0 != -1;
+        f1 = nc0 == ci;
+        for_id_pairs(A, Cc, K, [&](int32_t a, int32_t c) {
+          f0 += c == ai && a != -1;
+          f1 += c == ci;
+        });
+        if (ci == -1) f0 = f1 = 0;
       }
+    }
+    if (i < L) {
+      int32_t* out = side == 0 ? P.co_a : P.co_c;
       out[(g * L + i) * 2 + 0] = f0;
       out[(g * L + i) * 2 + 1] = f1;
     }
   }
+  __syncthreads();  // workgroup-uniform: every wavefront is here
+  if (wv == 0 && lane == 0 && P.co_pair != nullptr) P.co_pair[g] = static_cast<float>(*pairs);
 }
 
 // One wavefront per tile of queries.  No plan: a tile is m = 64/Bp consecutive
@@ -785,19 +788,28 @@ void recent_fused(Params P) {
       for (int p = sl; p < K - ncand; p += Bp) emit(p, -1, 0.0, -1);
     } else {
       if (v && K - nring + order >= 0) emit(K - nring + order, rid, rt, sl);
-      for (int p = sl; p < K - nring; p += Bp) {
-        if constexpr (CSR) {
-          if (p != sl) {
-            have0 = cbase + p >= s0;
-            if (have0) {
-              ct0 = P.c_times[cbase + p];
-              cid0 = P.c_ids[cbase + p];
-            }
+      if constexpr (CSR) {
+        if (sl < K - nring) emit(sl, have0 ? cid0 : -1, have0 ? ct0 : 0.0, have0 ? B + sl : -1);
+        // a window wider than the sub-group: kAhead entries loaded before the first goes out
+        constexpr int kAhead = NREG > 0 ? 1 : 4;
+        for (int q0 = sl + Bp; q0 < K - nring; q0 += kAhead * Bp) {
+          double t4[kAhead];
+          int32_t i4[kAhead];
+#pragma unroll
+          for (int u = 0; u < kAhead; ++u) {
+            const int p = q0 + u * Bp;
+            const bool in = p < K - nring && cbase + p >= s0;
+            t4[u] = in ? P.c_times[cbase + p] : 0.0;
+            i4[u] = in ? P.c_ids[cbase + p] : -1;
           }
-          emit(p, have0 ? cid0 : -1, have0 ? ct0 : 0.0, have0 ? B + p : -1);
-        } else {
-          emit(p, -1, 0.0, -1);
+#pragma unroll
+          for (int u = 0; u < kAhead; ++u) {
+            const int p = q0 + u * Bp;
+            if (p < K - nring) emit(p, i4[u], t4[u], cbase + p >= s0 ? B + p : -1);
+          }
         }
+      } else {
+        for (int p = sl; p < K - nring; p += Bp) emit(p, -1, 0.0, -1);
       }
     }
   } else {
@@ -947,15 +959,17 @@ void recent_fused(Params P) {
 
   // ---- co-occurrence of the plan group's (query 0, query 1) pair ----
   if (!TILES && P.co_mode != TGX_CO_NONE) {
+    int32_t* pairs = reinterpret_cast<int32_t*>(smem + P.te_bytes + P.off_pdt);  // wave 0's dt: its encodings are out
+    if (threadIdx.x == 0) *pairs = 0;
     __syncthreads();
     // workgroups from ev_b on (an event-major plan's tail) hold no pair
     const int64_t qa = g < P.ev_b ? query_of(P, g, 0) : -1;
     const int64_t qc = query_of(P, g, 1);
-    if (qa >= 0 && qc >= 0 && wv == 0) {
+    if (qa >= 0 && qc >= 0) {  // workgroup-uniform
       const int32_t* A = reinterpret_cast<const int32_t*>(smem + P.te_bytes + P.off_pid);
       const int32_t* Cc = reinterpret_cast<const int32_t*>(smem + P.te_bytes +
                                                           static_cast<size_t>(split) * P.wave_bytes + P.off_pid);
-      co_occurrence_pair(P, g, qa, qc, A, Cc, lane);
+      co_occurrence_pair(P, g, qa, qc, A, Cc, pairs, wv, static_cast<int>(blockDim.x) / kWave, lane);
     }
   }
 }
@@ -1317,6 +1331,106 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   }
 }
 
+// Co-occurrence of an event-major launch over the ids its gather wrote (the gather
+// ran tiled, csr_split, which shares nothing between queries): one pair per
+// workgroup, whose ids go through an LDS hash table with a counter per id and side,
+// so the work is linear in K (co_occurrence_pair's K^2 compares took 23.4 us for
+// 200 pairs at K = 512 here, 4.9 this way).  Counts as in co_occurrence_pair; the
+// masked counters hold the DyGFormer cross channel's: entries of one side at the
+// positions where the other side has one.
+constexpr int kCoThreads = kMaxWaves * kWave;
+constexpr int kCoOwn = (TGX_MAX_K + 1 + kCoThreads - 1) / kCoThreads;  // positions per thread
+constexpr int kCoBits = 11;
+constexpr int kCoSlots = 1 << kCoBits;
+static_assert(kCoSlots >= 2 * (TGX_MAX_K + 1) - 2, "slots for every id of both sides");
+__global__ __launch_bounds__(kCoThreads) void co_occurrence_events(Params P) {
+  __shared__ uint64_t key[kCoSlots];   // id with bit 32 set, 0: empty
+  __shared__ uint32_t cnt[kCoSlots];   // entries of A (low half) and C (high half) with the id
+  __shared__ uint32_t cntm[kCoSlots];  // those whose other side is not padding
+  __shared__ int pairs;
+  const int64_t g = blockIdx.x;
+  const int64_t qa = query_of(P, g, 0);
+  const int64_t qc = query_of(P, g, 1);
+  if (qa < 0 || qc < 0) return;  // workgroup-uniform
+  const bool freq = P.co_mode == TGX_CO_FREQ;
+  const int K = P.K;
+  const int lead = freq ? 0 : 1;  // DyGFormer sequences start with the query node
+  const int L = K + lead;
+  int32_t a[kCoOwn], c[kCoOwn];
+  int sa[kCoOwn], sc[kCoOwn];
+#pragma unroll
+  for (int u = 0; u < kCoOwn; ++u) {
+    const int i = static_cast<int>(threadIdx.x) + u * kCoThreads;
+    a[u] = c[u] = -1;
+    if (i >= lead && i < L) {
+      a[u] = P.o_ids[qa * K + (i - lead)];
+      c[u] = P.o_ids[qc * K + (i - lead)];
+    } else if (i < lead) {
+      a[u] = static_cast<int32_t>(query_node(P, qa));
+      c[u] = static_cast<int32_t>(query_node(P, qc));
+    }
+  }
+  for (int s = threadIdx.x; s < kCoSlots; s += kCoThreads) {
+    key[s] = 0;
+    cnt[s] = 0;
+    cntm[s] = 0;
+  }
+  if (threadIdx.x == 0) pairs = 0;
+  __syncthreads();
+  auto slot_of = [&](int32_t id) {
+    const uint64_t want = (uint64_t(1) << 32) | static_cast<uint32_t>(id);
+    int s = static_cast<int>((static_cast<uint32_t>(id) * 2654435761u) >> (32 - kCoBits));
+    while (true) {  // terminates: fewer ids than slots
+      const uint64_t old = atomicCAS(reinterpret_cast<unsigned long long*>(&key[s]), 0ull, want);
+      if (old == 0 || old == want) return s;
+      s = (s + 1) & (kCoSlots - 1);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < kCoOwn; ++u) {
+    const int i = static_cast<int>(threadIdx.x) + u * kCoThreads;
+    sa[u] = sc[u] = 0;
+    if (i < L && !(freq && a[u] == -1)) {
+      sa[u] = slot_of(a[u]);
+      atomicAdd(&cnt[sa[u]], 1u);
+      if (!freq && c[u] != -1) atomicAdd(&cntm[sa[u]], 1u);
+    }
+    if (i < L && !(freq && c[u] == -1)) {
+      sc[u] = slot_of(c[u]);
+      atomicAdd(&cnt[sc[u]], 1u << 16);
+      if (!freq && a[u] != -1) atomicAdd(&cntm[sc[u]], 1u << 16);
+    }
+  }
+  __syncthreads();
+  const int32_t nc = freq ? -1 : static_cast<int32_t>(query_node(P, qc));
+#pragma unroll
+  for (int u = 0; u < kCoOwn; ++u) {
+    const int i = static_cast<int>(threadIdx.x) + u * kCoThreads;
+    int2 fa = {0, 0}, fc = {0, 0};
+    int hits = 0;
+    if (i < L && a[u] != -1) {
+      const uint32_t x = cnt[sa[u]];
+      hits = static_cast<int>(x >> 16);
+      fa.x = static_cast<int>(x & 0xffffu);
+      fa.y = freq ? hits : static_cast<int>(cntm[sc[u]] & 0xffffu);
+      if (!freq) hits = i == 0 ? 0 : hits - (nc == a[u]);  // over the K sequences
+    }
+    if (i < L && c[u] != -1) {
+      const uint32_t x = cnt[sc[u]];
+      fc.x = static_cast<int>(freq ? x & 0xffffu : cntm[sa[u]] >> 16);
+      fc.y = static_cast<int>(x >> 16);
+    }
+    if (i < L) {
+      reinterpret_cast<int2*>(P.co_a)[g * L + i] = fa;
+      reinterpret_cast<int2*>(P.co_c)[g * L + i] = fc;
+    }
+    const int pc = __popcll(__ballot(hits > 0));
+    if ((threadIdx.x & (kWave - 1)) == 0 && pc > 0) atomicAdd(&pairs, pc);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && P.co_pair != nullptr) P.co_pair[g] = static_cast<float>(pairs);
+}
+
 // stand-alone co-occurrence (FREQ) over id rows: one wavefront per pair.  A
 // position is valid by its mask byte, or without masks when its id is not -1;
 // counts cover valid positions only (an id of -2^31 marks an invalid one in LDS:
@@ -1402,6 +1516,8 @@ struct Launch {
   bool window = false;  // csr_window runs the launch
   bool csr_split = false;  // csr_split runs it
   bool csr_ranges = false;  // in position ranges (K above 64)
+  bool co_after = false;  // co_occurrence_events counts after the gather, with co
+  Params co;
 };
 
 // |dt| below which every encoding argument fl32(fl32(dt w) + b) stays below
@@ -1432,7 +1548,7 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
     return fail(TGX_ERR_LIMIT, "tgx_recent: group=%d outside [1, %d]", a->group, TGX_MAX_GROUP);
   if (a->num_groups >= (int64_t(1) << 31))
     return fail(TGX_ERR_LIMIT, "tgx_recent: too many groups");
-  const int mode = a->plan != nullptr ? TGX_PLAN_LIST : a->plan_mode;
+  int mode = a->plan != nullptr ? TGX_PLAN_LIST : a->plan_mode;
   if (mode != TGX_PLAN_TILES && mode != TGX_PLAN_EVENTS && mode != TGX_PLAN_LIST)
     return fail(TGX_ERR_ARG, "tgx_recent: unknown plan_mode %d", a->plan_mode);
   if (mode == TGX_PLAN_LIST && a->plan == nullptr)
@@ -1598,6 +1714,20 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   P.co_pair = a->co_pair;
   P.status = a->status;
 
+  // An event-major launch over a CSR alone with K above 64 gathers as csr_split and
+  // counts its pairs afterwards: in the pair's workgroup every wave keeps all K
+  // positions in LDS (10 KB at K = 512), which leaves two waves per query, where
+  // csr_split runs eight (200 events at K = 512, 8-byte rows: 69.8 us in one launch,
+  // 30.3 in two; at K <= 64 the one launch is the faster).  Timed launches
+  // (timing_start) stay one kernel.
+  if (mode == TGX_PLAN_EVENTS && ring == nullptr && P.has_csr && a->k > kWave && a->co_mode != TGX_CO_NONE &&
+      a->timing_start == nullptr && (reinterpret_cast<uintptr_t>(a->co_a) & 7) == 0 &&
+      (reinterpret_cast<uintptr_t>(a->co_c) & 7) == 0) {
+    L.co_after = true;
+    L.co = P;
+    mode = P.plan_mode = TGX_PLAN_TILES;
+    P.co_mode = TGX_CO_NONE;
+  }
   const int K = a->k;
   // LDS of the rank: the ring's times, and with a CSR beside it K candidates (time
   // and id).  A tiled launch without a ring runs csr_window or csr_split (below);
@@ -1878,6 +2008,10 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
   }
 #undef TGX_PICK
   rc = check_launch(L.window ? "csr_window" : L.csr_split ? "csr_split" : "recent_fused");
+  if (rc == TGX_OK && L.co_after && L.co.ev_b > 0) {
+    hipLaunchKernelGGL(co_occurrence_events, dim3(static_cast<unsigned>(L.co.ev_b)), dim3(kCoThreads), 0, stream, L.co);
+    rc = check_launch("co_occurrence_events");
+  }
   if (rc != TGX_OK || !L.want_plan || L.fuse_plan) return rc;
   return launch_plan(L.pl, stream);  // batches beyond the fused plan's size
 }
