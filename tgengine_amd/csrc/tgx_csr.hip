@@ -374,7 +374,8 @@ __global__ __launch_bounds__(kThreads) void csr_node_keys(const int64_t* __restr
 // in 548 us (674 with the two arrays).  So tiles of `per` consecutive entries run
 // in the order of their first events: the busy nodes, which hold most of a skewed
 // stream's entries, then walk the stream together and share its lines, and runs of
-// kGatherSlice such tiles go to one XCD, for its L2: 353 us, and 23 us for the order.
+// kGatherSlice such tiles go to one XCD, for its L2: 345 us, and 23 us for the order
+// (tiles of 512 or 128 entries: 352 and 359).
 // A workgroup takes one tile, its permutation in LDS, and copies the rows as one
 // run of chunks, kGatherDepth per thread loaded before the first is stored,
 // whatever the row's width (314,948 entries with 688-byte rows: 118 -> 75 us
@@ -382,7 +383,7 @@ __global__ __launch_bounds__(kThreads) void csr_node_keys(const int64_t* __restr
 // the caches to the events (5 of 80 us on those).
 constexpr int kGatherDepth = 4;
 constexpr int kGatherChunks = kThreads * kGatherDepth;  // chunks a workgroup holds in flight
-constexpr int kGatherMost = 512;                        // entries per workgroup at most
+constexpr int kGatherMost = 256;                        // entries per workgroup at most
 constexpr int kXcds = 8;
 constexpr int kGatherSlice = 64;  // tiles of neighbouring events given to one XCD
 
