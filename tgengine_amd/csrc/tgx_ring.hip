@@ -48,8 +48,19 @@ constexpr int kCommitWaves = kThreads / kWave;
 constexpr int kWinBits = 8192;                 // bitmap window (indices)
 constexpr int kWinWords = kWinBits / 32;       // 256 words = 1 KB
 static_assert(kWinWords == kThreads, "one bitmap word per thread");
-constexpr int64_t kSmallGroupBlocks = 256;  // commit blocks for small groups (4 waves each)
-constexpr int64_t kLargeGroupBlocks = 64;   // four-launch commit blocks for large groups
+constexpr int kCountedGroup = 512;  // large groups ranked by counting up to this many entries
+constexpr int kListDepth = 16;      // list entries each thread loads before using them
+// four-launch commit blocks of the group roles, at most: a group is a chain of
+// dependent round trips, so the small groups (one wavefront each, four a block) get
+// as many wavefronts as the device holds (50,000 events of 172-d rows: 256 and 64
+// blocks took 81 us, 35 now with the ranking below)
+constexpr int64_t kSmallGroupBlocks = 2048;
+constexpr int64_t kLargeGroupBlocks = 256;
+// workgroups of the count and groups launches: each pays one global atomic per
+// distinct node (count) and three on the shared cursors (groups), so they are as
+// large as they go (256 threads, and cursor atomics per wavefront: 41 and 33 us for
+// 50,000 events, 21 and 5 now)
+constexpr int kTicketThreads = 1024;
 
 // (write_pos + off) % B for write_pos >= 0, 0 <= off < B
 __device__ __forceinline__ int64_t ring_slot(int64_t w, int off, int B) {
@@ -110,9 +121,9 @@ __device__ __forceinline__ void commit_diagnostics(const AppendParams& P, int ti
 }
 
 // ---- four-launch 1. count ----------------------------------------------------
-__global__ __launch_bounds__(kThreads) void append_count(PlanParams P) {
+__global__ __launch_bounds__(kTicketThreads) void append_count(PlanParams P) {
   __shared__ PlanLds L;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kTicketThreads + threadIdx.x;
   if (i == 0) {
     P.ctl[kCtlCursor] = 0;
     P.ctl[kCtlGroups] = 0;
@@ -138,8 +149,12 @@ __global__ __launch_bounds__(T) void fast_plan(PlanParams P) {
 }
 
 // ---- four-launch 2. groups --------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void append_groups(AppendParams P) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+__global__ __launch_bounds__(kTicketThreads) void append_groups(AppendParams P) {
+  // small groups, large groups and list space of each wavefront, then of the ones before it
+  __shared__ int wsum[3][kTicketThreads / kWave];
+  __shared__ int wbase[3];
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kTicketThreads + threadIdx.x;
+  const int wv = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   int64_t u = -1;
   int c = 0;
@@ -149,7 +164,7 @@ __global__ __launch_bounds__(kThreads) void append_groups(AppendParams P) {
   }
   const bool grp = c > 1;
   const bool big = c > kWave;
-  // wave-aggregated reservation of group ids and list space
+  // the workgroup's reservation of group ids and list space
   const uint64_t sm = __ballot(grp && !big);
   const uint64_t lm = __ballot(big);
   const int sum = grp ? c : 0;
@@ -159,18 +174,26 @@ __global__ __launch_bounds__(kThreads) void append_groups(AppendParams P) {
     const int y = __shfl_up(incl, off, kWave);
     if (lane >= off) incl += y;
   }
-  const int total = __shfl(incl, kWave - 1, kWave);
-  int sbase = 0, lgbase = 0, lbase = 0;
-  if ((sm | lm) != 0) {
-    if (lane == 0) {
-      if (sm) sbase = atomicAdd(&P.ctl[kCtlGroups], __popcll(sm));
-      if (lm) lgbase = atomicAdd(&P.ctl[kCtlLarge], __popcll(lm));
-      lbase = atomicAdd(&P.ctl[kCtlCursor], total);
-    }
-    sbase = __shfl(sbase, 0, kWave);
-    lgbase = __shfl(lgbase, 0, kWave);
-    lbase = __shfl(lbase, 0, kWave);
+  if (lane == kWave - 1) {
+    wsum[0][wv] = __popcll(sm);
+    wsum[1][wv] = __popcll(lm);
+    wsum[2][wv] = incl;
   }
+  __syncthreads();
+  if (threadIdx.x < 3) {
+    int total = 0;
+    for (int w = 0; w < kTicketThreads / kWave; ++w) {
+      const int x = wsum[threadIdx.x][w];
+      wsum[threadIdx.x][w] = total;
+      total += x;
+    }
+    const int word = threadIdx.x == 0 ? kCtlGroups : threadIdx.x == 1 ? kCtlLarge : kCtlCursor;
+    wbase[threadIdx.x] = total > 0 ? atomicAdd(&P.ctl[word], total) : 0;
+  }
+  __syncthreads();
+  const int sbase = wbase[0] + wsum[0][wv];
+  const int lgbase = wbase[1] + wsum[1][wv];
+  const int lbase = wbase[2] + wsum[2][wv];
   const uint64_t below = (uint64_t(1) << lane) - 1;
   if (grp && !big) P.groups[sbase + __popcll(sm & below)] = static_cast<int32_t>(u);
   if (big) P.large[lgbase + __popcll(lm & below)] = static_cast<int32_t>(u);
@@ -253,57 +276,97 @@ __device__ __forceinline__ void write_kept(const AppendParams& P, const int32_t*
     write_entry_meta(P, R[r], u * P.B + ring_slot(w, kept - 1 - r, P.B));
 }
 
-// one large group (c > 64) by the whole workgroup
+// One large group (c > 64) by the whole workgroup.  Up to kCountedGroup entries are
+// ranked by counting the later ones in LDS; a longer list over bitmap windows of
+// kWinBits entry indices, each ending at the last entry not yet seen (a node that
+// is only ever a source has none in the upper half of the batch), until `kept`
+// entries are found: one pass over the list per window, kListDepth loads in flight
+// per thread, and the set bits of a word give their ranks.  (Before, every group went through
+// the windows, with two passes of one load at a time: a hub holding 38% of 100,000
+// events kept its workgroup for 540 us, 34 now; a group of 100 entries needed
+// up to 16 windows.)
 template <int VEC>
 __device__ __forceinline__ void commit_large(const AppendParams& P, int64_t gid, uint32_t* bitmap,
-                                             int32_t* sfx, int32_t* R, int32_t* wsum) {
+                                             int32_t* listed, int32_t* R, int32_t* wsum) {
   const int wv = threadIdx.x / kWave;
   const int lane = threadIdx.x & (kWave - 1);
   const int t = threadIdx.x;
   const int64_t u = P.large[gid];
   const int c = P.cnt[u];
-  const int base = P.nbase[u];
+  const int32_t* list = P.list + P.nbase[u];
   const int kept = c < P.B ? c : P.B;
-  int64_t hi = P.n;
-  int carry = 0;
-  while (carry < kept && hi > 0) {  // uniform across the workgroup
-    const int64_t lo = hi > kWinBits ? hi - kWinBits : 0;
-    for (int q = t; q < kWinWords; q += kThreads) bitmap[q] = 0u;
-    __syncthreads();
-    for (int j = t; j < c; j += kThreads) {
-      const int64_t x = P.list[base + j];
-      if (x >= lo && x < hi) atomicOr(&bitmap[(x - lo) >> 5], 1u << ((x - lo) & 31));
-    }
-    __syncthreads();
-    // exclusive suffix over words: thread t owns word t (kWinWords == kThreads)
-    const int own = __popc(bitmap[t]);
-    int suf = own;
+  if (c <= kCountedGroup) {  // workgroup-uniform
+    int32_t x[kCountedGroup / kThreads];
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const int y = __shfl_down(suf, off, kWave);
-      if (lane + off < kWave) suf += y;
+    for (int r = 0; r < kCountedGroup / kThreads; ++r) {
+      const int j = r * kThreads + t;
+      x[r] = j < c ? list[j] : -1;  // -1 is later than none
+      listed[j] = x[r];
     }
-    if (lane == 0) wsum[wv] = suf;
     __syncthreads();
-    int later = 0, win_total = 0;
-    for (int w2 = 0; w2 < kCommitWaves; ++w2) {
-      if (w2 > wv) later += wsum[w2];
-      win_total += wsum[w2];
+    int e[kCountedGroup / kThreads] = {};
+    for (int j = 0; j < c; j += 4) {
+      const int4 y = *reinterpret_cast<const int4*>(listed + j);
+#pragma unroll
+      for (int r = 0; r < kCountedGroup / kThreads; ++r)
+        e[r] += (y.x > x[r]) + (y.y > x[r]) + (y.z > x[r]) + (y.w > x[r]);
     }
-    sfx[t] = later + suf - own;
+#pragma unroll
+    for (int r = 0; r < kCountedGroup / kThreads; ++r)
+      if (r * kThreads + t < c && e[r] < kept) R[e[r]] = x[r];
     __syncthreads();
-    for (int j = t; j < c; j += kThreads) {
-      const int64_t x = P.list[base + j];
-      if (x >= lo && x < hi) {
-        const int rel = static_cast<int>(x - lo);
-        const int word = rel >> 5;
-        const int e = carry + (__popc(bitmap[word] >> (rel & 31)) - 1) + sfx[word];
-        if (e < kept) R[e] = static_cast<int32_t>(x);
+  } else {
+    int carry = 0;
+    int32_t lo = static_cast<int32_t>(P.n), hi = lo;  // n < 2^30
+    while (true) {  // uniform across the workgroup; the first pass only finds the last entry
+      bitmap[t] = 0u;  // kWinWords == kThreads
+      __syncthreads();
+      int32_t top = -1;  // last entry before the window
+      for (int j0 = t; j0 < c; j0 += kListDepth * kThreads) {
+        int32_t x[kListDepth];
+#pragma unroll
+        for (int r = 0; r < kListDepth; ++r) x[r] = j0 + r * kThreads < c ? list[j0 + r * kThreads] : -1;
+#pragma unroll
+        for (int r = 0; r < kListDepth; ++r) {
+          if (x[r] >= lo && x[r] < hi) atomicOr(&bitmap[(x[r] - lo) >> 5], 1u << ((x[r] - lo) & 31));
+          if (x[r] < lo) top = x[r] > top ? x[r] : top;
+        }
       }
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) {
+        const int32_t y = __shfl_xor(top, off, kWave);
+        top = y > top ? y : top;
+      }
+      if (lane == 0) listed[wv] = top;
+      __syncthreads();
+      for (int w2 = 0; w2 < kCommitWaves; ++w2) top = listed[w2] > top ? listed[w2] : top;
+      // set bits in later words: thread t owns word t
+      uint32_t word = bitmap[t];
+      const int own = __popc(word);
+      int suf = own;
+#pragma unroll
+      for (int off = 1; off < kWave; off <<= 1) {
+        const int y = __shfl_down(suf, off, kWave);
+        if (lane + off < kWave) suf += y;
+      }
+      if (lane == 0) wsum[wv] = suf;
+      __syncthreads();
+      int later = 0, win_total = 0;
+      for (int w2 = 0; w2 < kCommitWaves; ++w2) {
+        if (w2 > wv) later += wsum[w2];
+        win_total += wsum[w2];
+      }
+      for (int e = carry + later + suf - own; word != 0 && e < kept; ++e) {
+        const int bit = 31 - __builtin_clz(word);
+        R[e] = lo + t * 32 + bit;
+        word &= ~(1u << bit);
+      }
+      carry += win_total;
+      __syncthreads();
+      if (carry >= kept || top < 0) break;
+      hi = top + 1;
+      lo = hi > kWinBits ? hi - kWinBits : 0;
     }
-    carry += win_total;
-    hi = lo;
-    __syncthreads();
   }
   const int64_t w = P.wp[u];
   write_kept<VEC>(P, R, u, kept, w, t, kThreads);
@@ -404,7 +467,7 @@ __device__ __forceinline__ void commit_small(const AppendParams& P, int64_t u, i
 template <int VEC>
 __global__ __launch_bounds__(kThreads) void append_commit(AppendParams P) {
   __shared__ uint32_t bitmap[kWinWords];
-  __shared__ int32_t sfx[kWinWords];                     // set bits in later words
+  __shared__ __align__(16) int32_t listed[kCountedGroup];  // a counted group's entries
   __shared__ int32_t rows[kCommitWaves][TGX_MAX_SLOTS];  // kept entry index by e
   __shared__ int32_t wsum[kCommitWaves];
   const int blk = static_cast<int>(blockIdx.x);
@@ -433,7 +496,7 @@ __global__ __launch_bounds__(kThreads) void append_commit(AppendParams P) {
   const int64_t nlarge = P.ctl[kCtlLarge];
   const int64_t gstride = static_cast<int64_t>(gridDim.x) - P.ga - P.gb;
   for (int64_t gid = blk - P.ga - P.gb; gid < nlarge; gid += gstride)  // workgroup-uniform
-    commit_large<VEC>(P, gid, bitmap, sfx, rows[0], wsum);
+    commit_large<VEC>(P, gid, bitmap, listed, rows[0], wsum);
 }
 
 // ---- two-launch 2. commit -------------------------------------------------------
@@ -596,10 +659,11 @@ int launch_plan(const PlanParams& P, hipStream_t stream) {
   AppendParams A{};
   static_cast<PlanParams&>(A) = P;
   A.nbase = P.lst;
-  hipLaunchKernelGGL(append_count, grid1, dim3(kThreads), 0, stream, static_cast<const PlanParams&>(A));
+  const dim3 gridt(static_cast<unsigned>((P.n + kTicketThreads - 1) / kTicketThreads));
+  hipLaunchKernelGGL(append_count, gridt, dim3(kTicketThreads), 0, stream, static_cast<const PlanParams&>(A));
   int rc = check_launch("append_count");
   if (rc) return rc;
-  hipLaunchKernelGGL(append_groups, grid1, dim3(kThreads), 0, stream, A);
+  hipLaunchKernelGGL(append_groups, gridt, dim3(kTicketThreads), 0, stream, A);
   if ((rc = check_launch("append_groups"))) return rc;
   hipLaunchKernelGGL(append_fill, grid1, dim3(kThreads), 0, stream, A);
   return check_launch("append_fill");

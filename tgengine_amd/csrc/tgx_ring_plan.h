@@ -24,9 +24,8 @@ namespace tgx {
 
 constexpr int kListCap = 8;                 // node-list entries per node (ring scratch)
 constexpr int64_t kFastMaxEntries = 32768;  // two-launch update up to this many entries
-constexpr int kPlanMaxThreads = 512;        // plan workgroups of 64..512 threads
-constexpr int kPlanMaxWaves = kPlanMaxThreads / kWave;
-constexpr int kPlanHashBits = 10;           // LDS hash of equal nodes, at most half full
+constexpr int kPlanMaxThreads = 1024;       // four-launch count workgroups
+constexpr int kPlanHashBits = 11;           // LDS hash of equal nodes, at most half full
 constexpr int kPlanHash = 1 << kPlanHashBits;
 static_assert(kPlanHash >= 2 * kPlanMaxThreads, "hash table at most half full");
 
@@ -68,7 +67,6 @@ struct PlanLds {
   int32_t hkey[kPlanHash];
   int32_t hcnt[kPlanHash];
   int32_t hbase[kPlanHash];
-  uint64_t wofs[kPlanMaxWaves + 1];
 };
 
 __device__ __forceinline__ int64_t entry_node(const int64_t* src, const int64_t* dst, int64_t i,
