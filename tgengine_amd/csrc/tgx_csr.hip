@@ -17,11 +17,10 @@
 // build order (a time-ordered stream); the time passes are skipped and the
 // kernels read an entry's node, neighbour, time and event from its event.
 #include "tgx_radix.h"
+#include "tgx_rows.h"
 
 namespace tgx {
 namespace {
-
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 // order-preserving image of a float64: -0.0 maps to +0.0 and every NaN to one
 // NaN above +inf, so ties are exactly the ties of a float comparison
@@ -397,11 +396,10 @@ __global__ __launch_bounds__(kThreads) void csr_tile_keys(const uint32_t* __rest
 template <int VEC>
 __global__ __launch_bounds__(kThreads) void csr_gather(
     const uint32_t* __restrict__ perm, int64_t n, const EventRec* __restrict__ rec, int pairs,
-    const int64_t* __restrict__ event, int64_t num_events, const uint8_t* __restrict__ feats, int nch,
+    const int64_t* __restrict__ event, int64_t num_events, const uint8_t* __restrict__ feats, int64_t row_bytes, int nch,
     uint32_t nch_magic, int per, const uint32_t* __restrict__ order, int64_t ntiles, int32_t* __restrict__ out_ids, double* __restrict__ out_times,
     int64_t* __restrict__ out_eids, uint8_t* __restrict__ out_feats, int32_t* __restrict__ status) {
-  using V = typename std::conditional<VEC == 16, u32x4,
-                                      typename std::conditional<VEC == 4, uint32_t, uint16_t>::type>::type;
+  using V = typename RowChunk<VEC>::T;
   __shared__ int64_t row[kGatherMost];  // an entry's feature row, -1: zeros
   int64_t tile = blockIdx.x;
   if (order != nullptr) {  // launch-uniform
@@ -428,27 +426,28 @@ __global__ __launch_bounds__(kThreads) void csr_gather(
   }
   if (out_feats == nullptr) return;  // launch-uniform
   __syncthreads();
-  const V* src = reinterpret_cast<const V*>(feats);
-  V* dst = reinterpret_cast<V*>(out_feats) + p0 * nch;
+  uint8_t* dst = out_feats + p0 * row_bytes;
   const int64_t total = static_cast<int64_t>(cnt) * nch;
   for (int64_t c0 = threadIdx.x; c0 < total; c0 += kGatherChunks) {
     V v[kGatherDepth];
+    int64_t at[kGatherDepth];
 #pragma unroll
     for (int u = 0; u < kGatherDepth; ++u) {
       const int64_t c = c0 + u * kThreads;
       v[u] = V{};
+      at[u] = 0;
       if (c < total) {
         // one entry per workgroup, or a dividend below 2^32 / nch
         const int e = per == 1 ? 0 : nch == 1 ? static_cast<int>(c) : static_cast<int>(__umulhi(static_cast<uint32_t>(c), nch_magic));
+        const int64_t off = chunk_at<VEC>(c - static_cast<int64_t>(e) * nch, row_bytes);
         const int64_t ev = row[e];
-        if (ev >= 0) v[u] = src[ev * nch + (c - static_cast<int64_t>(e) * nch)];
+        at[u] = e * row_bytes + off;
+        if (ev >= 0) v[u] = load_chunk<VEC>(feats + ev * row_bytes + off);
       }
     }
 #pragma unroll
-    for (int u = 0; u < kGatherDepth; ++u) {
-      const int64_t c = c0 + u * kThreads;
-      if (c < total) __builtin_nontemporal_store(v[u], dst + c);
-    }
+    for (int u = 0; u < kGatherDepth; ++u)
+      if (c0 + u * kThreads < total) store_chunk<VEC, true>(dst + at[u], v[u]);
   }
 }
 
@@ -596,14 +595,9 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
   hipLaunchKernelGGL(csr_offsets, dim3(static_cast<unsigned>(cdiv(N + 1, kThreads))), dim3(kThreads), 0,
                      stream, static_cast<const uint32_t*>(nk[ncur]), n, N, a->out_offsets);
   if ((rc = check_launch("csr_offsets"))) return rc;
-  int vec = 2;
   const bool fe = row_bytes > 0;
-  auto al = [](const void* p, unsigned m) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) & m) == 0; };
-  if (row_bytes % 16 == 0 && (!fe || (al(a->feats, 15) && al(a->out_feats, 15))))
-    vec = 16;
-  else if (row_bytes % 4 == 0 && (!fe || (al(a->feats, 3) && al(a->out_feats, 3))))
-    vec = 4;
-  const int64_t nch = fe ? row_bytes / vec : 1;
+  const int vec = fe ? row_vec(row_bytes, reinterpret_cast<uintptr_t>(a->feats) | reinterpret_cast<uintptr_t>(a->out_feats)) : 16;
+  const int64_t nch = fe ? row_chunks(row_bytes, vec) : 1;
   const int per = static_cast<int>(std::min<int64_t>(std::max<int64_t>(kGatherChunks / nch, 1), kGatherMost));
   const uint32_t magic = nch > 1 ? 0xffffffffu / static_cast<uint32_t>(nch) + 1u : 0u;
   const int64_t ntiles = cdiv(n, per);
@@ -630,12 +624,14 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
   auto gather = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(gblocks)), dim3(kThreads), 0, stream,
                        static_cast<const uint32_t*>(perm_in), n, static_cast<const EventRec*>(rec), pairs, a->event,
-                       a->num_events, static_cast<const uint8_t*>(a->feats), static_cast<int>(nch), magic, per, order, ntiles,
+                       a->num_events, static_cast<const uint8_t*>(a->feats), row_bytes, static_cast<int>(nch), magic, per, order, ntiles,
                        a->out_ids, a->out_times, a->out_eids, static_cast<uint8_t*>(fe ? a->out_feats : nullptr),
                        a->status);
   };
   if (vec == 16)
     gather(csr_gather<16>);
+  else if (vec == kAnyRow)
+    gather(csr_gather<kAnyRow>);
   else if (vec == 4)
     gather(csr_gather<4>);
   else

@@ -53,6 +53,7 @@
 
 #include "tgx_cos.h"
 #include "tgx_ring_plan.h"
+#include "tgx_rows.h"
 
 namespace tgx {
 namespace {
@@ -140,21 +141,6 @@ struct Params {
   double c_tmax;  // largest non-NaN CSR time (+inf: unknown)
   int wg_parts;   // csr_split: workgroups per query (1: a workgroup holds whole queries)
   int te_nt;      // csr_split: nontemporal encoding stores (rows of at least kNtRowBytes)
-};
-
-template <int VEC>
-struct Vec;
-template <>
-struct Vec<16> {
-  using T = u32x4;
-};
-template <>
-struct Vec<4> {
-  using T = uint32_t;
-};
-template <>
-struct Vec<2> {
-  using T = uint16_t;
 };
 
 __constant__ double kRevTableDev[][2] = {TGX_REV_TABLE_ROWS};
@@ -529,7 +515,7 @@ __device__ __forceinline__ void co_occurrence_pair(const Params& P, int64_t g, i
 // event-plan CSR copies with rows through memory; 7 for the rest, where it keeps a
 // private segment (a scalar spill's) out of the kernel.
 template <int VEC, int NREG, bool TILES, bool CSR>
-constexpr int kWavesPerEu = TILES ? (VEC == 16 || CSR ? 1 : 7)
+constexpr int kWavesPerEu = TILES ? (VEC == 16 || VEC == kAnyRow || CSR ? 1 : 7)
                                   : CSR ? (NREG > 0 || VEC == 2 ? 7 : 1) : (NREG > 0 ? 7 : 8);
 
 // TILES: the launch's plan mode is TGX_PLAN_TILES (no event or list plan, so no
@@ -540,7 +526,7 @@ constexpr int kWavesPerEu = TILES ? (VEC == 16 || CSR ? 1 : 7)
 template <int VEC, int NREG, bool TILES, bool CSR>
 __global__ __launch_bounds__(kMaxWaves * kWave) __attribute__((amdgpu_waves_per_eu(kWavesPerEu<VEC, NREG, TILES, CSR>)))
 void recent_fused(Params P) {
-  using VT = typename Vec<VEC>::T;
+  using VT = typename RowChunk<VEC>::T;
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
@@ -908,6 +894,7 @@ void recent_fused(Params P) {
       constexpr int kDepth = TILES ? kCopyDepth : 2 * kCopyDepth;
       for (int idx0 = part * kWave; idx0 < total; idx0 += kDepth * ostride) {
         VT v4[kDepth];
+        int at[kDepth];  // kAnyRow: byte offset in the wave's output rows
 #pragma unroll
         for (int u = 0; u < kDepth; ++u) {
           const int idx = idx0 + u * ostride + lane;
@@ -917,17 +904,27 @@ void recent_fused(Params P) {
             const int c = idx - gp * nch;
             const int hh = static_cast<int>(dk.div(gp));
             const int code = pcode[gp];
+            const int rb = static_cast<int>(P.row_bytes);
+            if constexpr (VEC == kAnyRow) at[u] = gp * rb + chunk_at<VEC>(c, rb);
             if (code >= 0) {
               const uint8_t* src = !CSR || code < B ? P.r_feats + (tur[hh] * B + code) * P.row_bytes
                                                     : P.c_feats + (tcb[hh] + (code - B)) * P.row_bytes;
-              v4[u] = reinterpret_cast<const VT*>(src)[c];
+              if constexpr (VEC == kAnyRow)
+                v4[u] = load_chunk<VEC>(src + chunk_at<VEC>(c, rb));
+              else
+                v4[u] = reinterpret_cast<const VT*>(src)[c];
             }
           }
         }
 #pragma unroll
         for (int u = 0; u < kDepth; ++u) {
           const int idx = idx0 + u * ostride + lane;
-          if (idx < total) put<true>(of + idx, v4[u]);
+          if (idx < total) {
+            if constexpr (VEC == kAnyRow)
+              store_chunk<VEC, true>(P.o_feats + r0 * P.row_bytes + at[u], v4[u]);
+            else
+              put<true>(of + idx, v4[u]);
+          }
         }
       }
     }
@@ -1154,7 +1151,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
 // away 20 MB of rows and took 17.4 us, 16.1 now.
 template <int VEC, bool RANGES>
 __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
-  using VT = typename Vec<VEC>::T;
+  using VT = typename RowChunk<VEC>::T;
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
@@ -1225,7 +1222,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   const int nch = P.nch;
   const int total = np * nch;  // chunks of the wave's positions
   const FastDiv dv(nch, P.fd_c);
-  const VT* crow = reinterpret_cast<const VT*>(P.c_feats);
+  const int rb = static_cast<int>(P.row_bytes);
   VT v[kCopyDepth];
 #pragma unroll
   for (int u = 0; u < kCopyDepth; ++u) v[u] = VT{};
@@ -1250,7 +1247,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
       if (fe && live && idx < total) {
         const int pl = static_cast<int>(dv.div(idx));
         const int64_t x = s1 - K + p0 + pl;
-        if (x >= s0) v[u] = crow[x * nch + (idx - pl * nch)];
+        if (x >= s0) v[u] = load_chunk<VEC>(P.c_feats + x * P.row_bytes + chunk_at<VEC>(idx - pl * nch, rb));
       }
     }
     if (!RANGES) tl = __shfl(t, K - 1);  // entry s1 - 1 whenever the window is not empty
@@ -1273,7 +1270,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   if (q >= 0 && np > 0) {  // wave-uniform
     // ---- feature rows of the wave's positions ----
     if (fe) {
-      VT* of = reinterpret_cast<VT*>(P.o_feats) + (q * K + p0) * nch;
+      uint8_t* of = P.o_feats + (q * K + p0) * P.row_bytes;
       for (int idx0 = off; idx0 < total; idx0 += kCopyDepth * cstride) {
         if (idx0 != off || reload) {
 #pragma unroll
@@ -1282,14 +1279,22 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
             v[u] = VT{};
             if (idx < total) {
               const int pl = static_cast<int>(dv.div(idx));
-              if (p0 + pl >= K - take) v[u] = crow[(base + p0 + pl) * nch + (idx - pl * nch)];
+              if (p0 + pl >= K - take)
+                v[u] = load_chunk<VEC>(P.c_feats + (base + p0 + pl) * P.row_bytes + chunk_at<VEC>(idx - pl * nch, rb));
             }
           }
         }
 #pragma unroll
         for (int u = 0; u < kCopyDepth; ++u) {
           const int idx = idx0 + u * cstride + lane;
-          if (idx < total) put<true>(of + idx, v[u]);
+          if (idx < total) {
+            if constexpr (VEC == kAnyRow) {
+              const int pl = static_cast<int>(dv.div(idx));
+              store_chunk<VEC, true>(of + pl * rb + chunk_at<VEC>(idx - pl * nch, rb), v[u]);
+            } else {
+              store_chunk<VEC, true>(of + static_cast<int64_t>(idx) * VEC, v[u]);
+            }
+          }
         }
       }
     }
@@ -1818,21 +1823,21 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   size_t lds = static_cast<size_t>(P.te_bytes) + static_cast<size_t>(waves) * P.wave_bytes;
   if (lds > 160 * 1024) return fail(TGX_ERR_LIMIT, "tgx_recent: %zu bytes of LDS needed", lds);
 
-  int vec = 2;
   const bool fe = a->out_feats != nullptr && P.row_bytes > 0;
-  auto al = [](const void* p, unsigned m) { return p == nullptr || (reinterpret_cast<uintptr_t>(p) & m) == 0; };
-  if (P.row_bytes % 16 == 0 && (!fe || (al(P.r_feats, 15) && al(P.c_feats, 15) && al(P.o_feats, 15))))
-    vec = 16;
-  else if (P.row_bytes % 4 == 0 && (!fe || (al(P.r_feats, 3) && al(P.c_feats, 3) && al(P.o_feats, 3))))
-    vec = 4;
-  P.nch = static_cast<int>(P.row_bytes / vec);
+  const uintptr_t rows_at = fe ? reinterpret_cast<uintptr_t>(P.r_feats) | reinterpret_cast<uintptr_t>(P.c_feats) |
+                                     reinterpret_cast<uintptr_t>(P.o_feats)
+                               : 0;
+  const int vec = row_vec(P.row_bytes, rows_at);
+  P.nch = static_cast<int>(row_chunks(P.row_bytes, vec));
+  // the limit below in the widest chunks that the rows' alignment allows
+  const uint64_t unit = vec != kAnyRow ? vec : P.row_bytes % 4 == 0 && (rows_at & 3) == 0 ? 4 : 2;
+  const uint64_t units = static_cast<uint64_t>(P.row_bytes) / unit;
   // FastDiv(n) is exact for x * n < 2^32; its largest dividends: K * nch
   // feature chunks (divided by nch), m*K*d_t encodings (by d_t or d_t / 4) and
   // m*K positions (by K)
-  if (static_cast<uint64_t>(K) * static_cast<uint64_t>(P.nch) * static_cast<uint64_t>(P.nch) >=
-      (uint64_t(1) << 32))
+  if (static_cast<uint64_t>(K) * units * units >= (uint64_t(1) << 32))
     return fail(TGX_ERR_LIMIT, "tgx_recent: k=%d with %lld-byte rows (%d chunks of %d bytes) exceeds "
-                "the kernel's index range", K, (long long)P.row_bytes, P.nch, vec);
+                "the kernel's index range", K, (long long)P.row_bytes, (int)units, (int)unit);
   P.fd_k = FastDiv::magic(static_cast<uint32_t>(P.K));
   P.fd_q = FastDiv::magic(static_cast<uint32_t>(P.d_t / 4));
   P.fd_d = FastDiv::magic(static_cast<uint32_t>(P.d_t));
@@ -1925,21 +1930,25 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
     const void* fns[] = {reinterpret_cast<const void*>(recent_fused<16, 0, false, false>),
                          reinterpret_cast<const void*>(recent_fused<16, 2, false, false>),
                          reinterpret_cast<const void*>(recent_fused<16, 4, false, false>),
+                         reinterpret_cast<const void*>(recent_fused<kAnyRow, 0, false, false>),
                          reinterpret_cast<const void*>(recent_fused<4, 0, false, false>),
                          reinterpret_cast<const void*>(recent_fused<2, 0, false, false>),
                          reinterpret_cast<const void*>(recent_fused<16, 0, false, true>),
                          reinterpret_cast<const void*>(recent_fused<16, 2, false, true>),
                          reinterpret_cast<const void*>(recent_fused<16, 4, false, true>),
+                         reinterpret_cast<const void*>(recent_fused<kAnyRow, 0, false, true>),
                          reinterpret_cast<const void*>(recent_fused<4, 0, false, true>),
                          reinterpret_cast<const void*>(recent_fused<2, 0, false, true>),
                          reinterpret_cast<const void*>(recent_fused<16, 0, true, false>),
                          reinterpret_cast<const void*>(recent_fused<16, 2, true, false>),
                          reinterpret_cast<const void*>(recent_fused<16, 4, true, false>),
+                         reinterpret_cast<const void*>(recent_fused<kAnyRow, 0, true, false>),
                          reinterpret_cast<const void*>(recent_fused<4, 0, true, false>),
                          reinterpret_cast<const void*>(recent_fused<2, 0, true, false>),
                          reinterpret_cast<const void*>(recent_fused<16, 0, true, true>),
                          reinterpret_cast<const void*>(recent_fused<16, 2, true, true>),
                          reinterpret_cast<const void*>(recent_fused<16, 4, true, true>),
+                         reinterpret_cast<const void*>(recent_fused<kAnyRow, 0, true, true>),
                          reinterpret_cast<const void*>(recent_fused<4, 0, true, true>),
                          reinterpret_cast<const void*>(recent_fused<2, 0, true, true>)};
     for (const void* f : fns)
@@ -1982,6 +1991,8 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
     if (L.csr_ranges) {
       if (L.vec == 16)
         launch(csr_split<16, true>);
+      else if (L.vec == kAnyRow)
+        launch(csr_split<kAnyRow, true>);
       else if (L.vec == 4)
         launch(csr_split<4, true>);
       else
@@ -1989,6 +2000,8 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
     } else {
       if (L.vec == 16)
         launch(csr_split<16, false>);
+      else if (L.vec == kAnyRow)
+        launch(csr_split<kAnyRow, false>);
       else if (L.vec == 4)
         launch(csr_split<4, false>);
       else
@@ -2001,6 +2014,8 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
       TGX_PICK(16, 4);
     else
       TGX_PICK(16, 0);
+  } else if (L.vec == kAnyRow) {
+    TGX_PICK(kAnyRow, 0);
   } else if (L.vec == 4) {
     TGX_PICK(4, 0);
   } else {

@@ -34,6 +34,7 @@
 // Every path writes the kept entries and advances write_pos.  Feature rows move
 // as 16-byte vectors when the row allows it.
 #include "tgx_ring_plan.h"
+#include "tgx_rows.h"
 
 #include <algorithm>
 #include <mutex>
@@ -77,25 +78,11 @@ __device__ __forceinline__ void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int VEC>
-struct VecT;
-template <>
-struct VecT<16> {
-  using T = uint4;
-};
-template <>
-struct VecT<4> {
-  using T = uint32_t;
-};
-template <>
-struct VecT<2> {
-  using T = uint16_t;
-};
-
 struct AppendParams : PlanParams {
   const uint8_t* feat;  // [b, row_bytes] or null (zero rows)
   int B;
   int64_t row_bytes;
+  int nch;  // chunks of a row (tgx_rows.h)
   int64_t eid_base;
   int32_t* ids;
   double* times;
@@ -229,8 +216,9 @@ constexpr int kKeptDepth = 4;
 template <int VEC>
 __device__ __forceinline__ void write_kept(const AppendParams& P, const int32_t* R, int64_t u,
                                            int kept, int64_t w, int first, int stride) {
-  using V = typename VecT<VEC>::T;
-  const int nv = static_cast<int>(P.row_bytes / VEC);
+  using V = typename RowChunk<VEC>::T;
+  const int nv = P.nch;
+  const int rb = static_cast<int>(P.row_bytes);
   const int total = kept * nv;
   // the thread's first row: id, time, edge id (loaded with the first chunks)
   int32_t m_id = 0;
@@ -245,7 +233,7 @@ __device__ __forceinline__ void write_kept(const AppendParams& P, const int32_t*
   }
   for (int f0 = first; f0 < total || m_slot >= 0; f0 += kKeptDepth * stride) {
     V v[kKeptDepth];
-    V* dp[kKeptDepth];
+    uint8_t* dp[kKeptDepth];
 #pragma unroll
     for (int k = 0; k < kKeptDepth; ++k) {
       const int f = f0 + k * stride;
@@ -257,8 +245,9 @@ __device__ __forceinline__ void write_kept(const AppendParams& P, const int32_t*
         const int64_t i = R[r];
         const int64_t e = i < P.b ? i : i - P.b;
         const int64_t slot = u * P.B + ring_slot(w, kept - 1 - r, P.B);
-        dp[k] = reinterpret_cast<V*>(P.feats + slot * P.row_bytes) + cch;
-        if (P.feat != nullptr) v[k] = reinterpret_cast<const V*>(P.feat + e * P.row_bytes)[cch];
+        const int off = chunk_at<VEC>(cch, rb);
+        dp[k] = P.feats + slot * P.row_bytes + off;
+        if (P.feat != nullptr) v[k] = load_chunk<VEC>(P.feat + e * P.row_bytes + off);
       }
     }
     if (m_slot >= 0) {
@@ -269,7 +258,7 @@ __device__ __forceinline__ void write_kept(const AppendParams& P, const int32_t*
     }
 #pragma unroll
     for (int k = 0; k < kKeptDepth; ++k)
-      if (dp[k] != nullptr) *dp[k] = v[k];
+      if (dp[k] != nullptr) store_chunk<VEC, false>(dp[k], v[k]);
   }
   // rows beyond the first of this thread (only when kept > stride)
   for (int r = first + stride; r < kept; r += stride)
@@ -385,8 +374,9 @@ __device__ __forceinline__ void commit_large(const AppendParams& P, int64_t gid,
 // in rounds of kKeptDepth loads, then stores.
 template <int VEC>
 __device__ __forceinline__ void commit_singletons(const AppendParams& P, int blk) {
-  using V = typename VecT<VEC>::T;
-  const int nv = static_cast<int>(P.row_bytes / VEC);
+  using V = typename RowChunk<VEC>::T;
+  const int nv = P.nch;
+  const int rb = static_cast<int>(P.row_bytes);
   const int tpe = 1 << P.tpe_log2;
   const int epb = static_cast<int>(blockDim.x) >> P.tpe_log2;
   const int64_t i = static_cast<int64_t>(blk) * epb + (threadIdx.x >> P.tpe_log2);
@@ -396,12 +386,12 @@ __device__ __forceinline__ void commit_singletons(const AppendParams& P, int blk
   // a singleton, so the role costs two round trips
   const int64_t e = i < P.b ? i : i - P.b;
   const int64_t u = entry_node(P.src, P.dst, i, P.b);
-  const V* srow = reinterpret_cast<const V*>(P.feat + e * P.row_bytes);
+  const uint8_t* srow = P.feat + e * P.row_bytes;
   V v[kKeptDepth];
 #pragma unroll
   for (int k = 0; k < kKeptDepth; ++k) {
     const int c = l + k * tpe;
-    v[k] = (P.feat != nullptr && c < nv) ? srow[c] : V{};
+    v[k] = (P.feat != nullptr && c < nv) ? load_chunk<VEC>(srow + chunk_at<VEC>(c, rb)) : V{};
   }
   int32_t other = 0;
   double tm = 0.0;
@@ -415,22 +405,22 @@ __device__ __forceinline__ void commit_singletons(const AppendParams& P, int blk
   const int64_t w = P.wp[u];
   if (cn != 1) return;
   const int64_t slot = u * P.B + ring_slot(w, 0, P.B);
-  V* drow = reinterpret_cast<V*>(P.feats + slot * P.row_bytes);
+  uint8_t* drow = P.feats + slot * P.row_bytes;
 #pragma unroll
   for (int k = 0; k < kKeptDepth; ++k) {
     const int c = l + k * tpe;
-    if (c < nv) drow[c] = v[k];
+    if (c < nv) store_chunk<VEC, false>(drow + chunk_at<VEC>(c, rb), v[k]);
   }
   for (int c0 = l + kKeptDepth * tpe; c0 < nv; c0 += kKeptDepth * tpe) {
 #pragma unroll
     for (int k = 0; k < kKeptDepth; ++k) {
       const int c = c0 + k * tpe;
-      v[k] = (P.feat != nullptr && c < nv) ? srow[c] : V{};
+      v[k] = (P.feat != nullptr && c < nv) ? load_chunk<VEC>(srow + chunk_at<VEC>(c, rb)) : V{};
     }
 #pragma unroll
     for (int k = 0; k < kKeptDepth; ++k) {
       const int c = c0 + k * tpe;
-      if (c < nv) drow[c] = v[k];
+      if (c < nv) store_chunk<VEC, false>(drow + chunk_at<VEC>(c, rb), v[k]);
     }
   }
   if (l == 0) {
@@ -510,9 +500,10 @@ __global__ __launch_bounds__(kThreads) void append_commit(AppendParams P) {
 constexpr int kKeptThreads = 256;
 template <int VEC>
 __global__ __launch_bounds__(kKeptThreads) void kept_commit(AppendParams P) {
-  using V = typename VecT<VEC>::T;
+  using V = typename RowChunk<VEC>::T;
   if (blockIdx.x == 0 && threadIdx.x == 0) commit_diagnostics(P, kCtlKTime, kCtlKBad);
-  const int nv = static_cast<int>(P.row_bytes / VEC);
+  const int nv = P.nch;
+  const int rb = static_cast<int>(P.row_bytes);
   const int tpe = 1 << P.tpe_log2;
   const int epb = kKeptThreads >> P.tpe_log2;
   const int64_t i = static_cast<int64_t>(blockIdx.x) * epb + (threadIdx.x >> P.tpe_log2);
@@ -521,12 +512,12 @@ __global__ __launch_bounds__(kKeptThreads) void kept_commit(AppendParams P) {
   const longlong2 kr = reinterpret_cast<const longlong2*>(P.krec)[i];
   const int64_t e = i < P.b ? i : i - P.b;
   const int64_t u = entry_node(P.src, P.dst, i, P.b);
-  const V* srow = reinterpret_cast<const V*>(P.feat + e * P.row_bytes);
+  const uint8_t* srow = P.feat + e * P.row_bytes;
   V v[kKeptDepth];
 #pragma unroll
   for (int k = 0; k < kKeptDepth; ++k) {
     const int c = l + k * tpe;
-    v[k] = (P.feat != nullptr && c < nv) ? srow[c] : V{};
+    v[k] = (P.feat != nullptr && c < nv) ? load_chunk<VEC>(srow + chunk_at<VEC>(c, rb)) : V{};
   }
   int32_t other = 0;
   double tm = 0.0;
@@ -536,22 +527,22 @@ __global__ __launch_bounds__(kKeptThreads) void kept_commit(AppendParams P) {
   }
   if (kr.x >= 0) {
     const int64_t slot = u * P.B + kr.x;
-    V* drow = reinterpret_cast<V*>(P.feats + slot * P.row_bytes);
+    uint8_t* drow = P.feats + slot * P.row_bytes;
 #pragma unroll
     for (int k = 0; k < kKeptDepth; ++k) {
       const int c = l + k * tpe;
-      if (c < nv) drow[c] = v[k];
+      if (c < nv) store_chunk<VEC, false>(drow + chunk_at<VEC>(c, rb), v[k]);
     }
     for (int c0 = l + kKeptDepth * tpe; c0 < nv; c0 += kKeptDepth * tpe) {
 #pragma unroll
       for (int k = 0; k < kKeptDepth; ++k) {
         const int c = c0 + k * tpe;
-        v[k] = (P.feat != nullptr && c < nv) ? srow[c] : V{};
+        v[k] = (P.feat != nullptr && c < nv) ? load_chunk<VEC>(srow + chunk_at<VEC>(c, rb)) : V{};
       }
 #pragma unroll
       for (int k = 0; k < kKeptDepth; ++k) {
         const int c = c0 + k * tpe;
-        if (c < nv) drow[c] = v[k];
+        if (c < nv) store_chunk<VEC, false>(drow + chunk_at<VEC>(c, rb), v[k]);
       }
     }
     if (l == 0) {
@@ -699,13 +690,9 @@ int setup_append(const char* who, const tgx_ring* ring, const int64_t* src, cons
   P.nbase = P.lst;
   P.status = status;
 
-  vec = 2;
-  if (P.row_bytes % 16 == 0 && aligned16(ring->feats) && (feat == nullptr || aligned16(feat)))
-    vec = 16;
-  else if (P.row_bytes % 4 == 0 && (reinterpret_cast<uintptr_t>(ring->feats) & 3u) == 0 &&
-           (feat == nullptr || (reinterpret_cast<uintptr_t>(feat) & 3u) == 0))
-    vec = 4;
-  const int64_t nchunks = P.row_bytes / vec;
+  vec = row_vec(P.row_bytes, reinterpret_cast<uintptr_t>(ring->feats) | reinterpret_cast<uintptr_t>(feat));
+  const int64_t nchunks = row_chunks(P.row_bytes, vec);
+  P.nch = static_cast<int>(nchunks);
   int tpe_log2 = 0;
   // lanes per singleton entry: one chunk each up to 16 lanes, then several per lane
   while ((int64_t(1) << tpe_log2) < nchunks && tpe_log2 < 4) ++tpe_log2;
@@ -735,6 +722,9 @@ int launch_commit(const AppendParams& P, int vec, hipStream_t stream) {
   switch (vec) {
     case 16:
       launch_commit_vec<16>(P, stream);
+      break;
+    case kAnyRow:
+      launch_commit_vec<kAnyRow>(P, stream);
       break;
     case 4:
       launch_commit_vec<4>(P, stream);
