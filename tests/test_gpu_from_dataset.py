@@ -59,3 +59,37 @@ def test_from_dataset_refusals():
         TemporalGraph.from_dataset(src, dst, time, feat[:20], 50)
     with pytest.raises(IndexError):
         TemporalGraph.from_dataset(src, dst, time, feat, 5)
+
+
+@pytest.mark.parametrize("order", ["strict", "ties", "shuffled"])
+def test_from_dataset_leaves_its_arrays_to_other_streams(order):
+    """When from_dataset returns, nothing reads its arrays any more: a second stream
+    that never waits for the caller's refills them at once, and arrays allocated on a
+    loader's stream go back to that stream's pool and are handed out again."""
+    E, N, d = 400_000, 5_000, 64
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    src = torch.randint(0, N, (E,), generator=gen, device="cuda")
+    dst = torch.randint(0, N, (E,), generator=gen, device="cuda")
+    time = torch.arange(E, dtype=torch.float64, device="cuda") + 7.0
+    if order == "ties":
+        time = torch.floor(time / 3)
+    elif order == "shuffled":
+        time = time.view(-1, 100).flip(1).reshape(-1).contiguous()
+    feat = torch.randn(E, d, generator=gen, device="cuda")
+    want = TemporalGraph.from_dataset(src.cpu(), dst.cpu(), time.cpu(), feat.cpu(), N, track_edge_ids=True)
+    other = torch.cuda.Stream()
+    for release in (False, True):
+        with torch.cuda.stream(other):
+            arrays = [x.clone() for x in (src, dst, time, feat)]
+        torch.cuda.current_stream().wait_stream(other)
+        g = TemporalGraph.from_dataset(*arrays, N, track_edge_ids=True)
+        assert torch.cuda.current_stream().query()  # the build is over
+        with torch.cuda.stream(other):
+            if release:
+                del arrays
+                arrays = [torch.empty_like(x) for x in (src, dst, time, feat)]
+            for x in arrays:
+                x.zero_()
+        torch.cuda.synchronize()
+        for name in ("_offsets", "_nbr_ids", "_nbr_times", "_nbr_feats", "_nbr_eids"):
+            assert torch.equal(getattr(g, name), getattr(want, name)), name

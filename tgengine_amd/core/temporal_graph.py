@@ -408,9 +408,10 @@ class TemporalGraph:
     def _build_adopt(self, src: Tensor, dst: Tensor, time: Tensor, feat: Optional[Tensor], call: int) -> bool:
         """Take the events of advance() calls of ``call`` events each as the event
         buffers of an empty graph, without copying device arrays that already have
-        the buffers' layout: for a caller that freezes the graph before it returns,
-        so that the arrays are read in its own stream's order.  False, with nothing
-        taken, where advance() would refuse one of the calls."""
+        the buffers' layout: for a caller that freezes the graph and waits for the
+        build before it returns, since until then the build reads the arrays where
+        they are, and whoever owns them may reuse them on any stream.  False, with
+        nothing taken, where advance() would refuse one of the calls."""
         n = int(src.shape[0])
         if dst.shape[0] < n or time.shape[0] < n or (feat is not None and feat.shape[0] < n):
             return False
@@ -424,7 +425,7 @@ class TemporalGraph:
                        "time": _as(arrays[2], torch.float64, dev)}
         if feat is not None and self.edge_feat_dim > 0:
             self._build["feat"] = feat.detach()
-        self._build_starts = list(range(0, n, call))
+        self._build_starts = range(0, n, call)
         self._build_n = n
         self._num_edges = n
         return True
@@ -464,7 +465,11 @@ class TemporalGraph:
             L = _lib.lib()
             ws = torch.empty(max(int(L.tgx_csr_build_workspace_size(n)), int(L.tgx_csr_scan_workspace_size())),
                              dtype=torch.uint8, device=dev)
-            call_starts = torch.tensor(self._build_starts, dtype=torch.int64).to(dev)
+            starts = self._build_starts
+            if isinstance(starts, range):  # regular calls: no upload, and no wait for it
+                call_starts = torch.arange(starts.start, starts.stop, starts.step, dtype=torch.int64, device=dev)
+            else:
+                call_starts = torch.tensor(starts, dtype=torch.int64).to(dev)
             scan = torch.empty(4, dtype=torch.int64, device=dev)
             _lib.check(L.tgx_csr_scan(src.data_ptr(), dst.data_ptr(), tt.data_ptr(), E, call_starts.data_ptr(),
                                       call_starts.numel(), scan.data_ptr(), ws.data_ptr(), ws.numel(),
@@ -725,12 +730,19 @@ class TemporalGraph:
         graph = cls(num_nodes, edge_feat_dim=d_edge, device=device, **kwargs)
         chunk = 10000
         n = src.shape[0]
-        # all the calls' events at once, frozen right below: 157,474 events with
-        # 172-d rows went through 82 copies and took 580 us with the freeze, 154 without
-        if cls.advance is not TemporalGraph.advance or not graph._build_adopt(src, dst, time, edge_feat, chunk):
-            for s in range(0, n, chunk):
-                e = min(s + chunk, n)
-                graph.advance(src[s:e], dst[s:e], time[s:e],
-                              edge_feat[s:e] if edge_feat is not None else None)
+        # all the calls' events at once, frozen where they are: 157,474 events with
+        # 172-d rows went through 82 copies and took 580 us with the freeze, 200 this
+        # way (157 without the wait, with the next call's host work beside the build)
+        if cls.advance is TemporalGraph.advance and graph._build_adopt(src, dst, time, edge_feat, chunk):
+            try:
+                graph.freeze_csr()
+            finally:
+                # the arrays are the caller's again, to refill or release on any stream
+                torch.cuda.current_stream(graph.device).synchronize()
+            return graph
+        for s in range(0, n, chunk):
+            e = min(s + chunk, n)
+            graph.advance(src[s:e], dst[s:e], time[s:e],
+                          edge_feat[s:e] if edge_feat is not None else None)
         graph.freeze_csr()
         return graph
