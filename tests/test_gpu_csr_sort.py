@@ -3,12 +3,15 @@ changes, bit for bit against the oracle: runs of equal times and calls that star
 end and lie inside and across the 2,048-event tiles of the segment search; sorts of
 one and several tiles per workgroup (2M keys, 2,048- and 4,096-key tiles); one to
 three digit passes; entry counts on both sides of the event-ordered gather (2^20)."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 from oracle import spec as O
 from tgengine_amd import TemporalGraph
+from tgengine_amd.core import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -63,3 +66,45 @@ def test_sort_and_gather_sizes(E, N, d, order):
         time = time.reshape(-1, 100)[:, ::-1].reshape(-1).copy()
     g = _check(N, d, [0, E // 3, E], src, dst, time)
     assert g._csr_build_mode == {"strict": "pairs", "ties": "runs", "shuffled": "sort"}[order]
+
+
+def _by_call(N, src, dst, time, call, flags=0):
+    """tgx_csr_build of the events of advance() calls of ``call`` events: (build, outputs)."""
+    L, E = _lib.lib(), src.numel()
+    empty = lambda n, dt: torch.empty(n, dtype=dt, device="cuda")  # noqa: E731
+    starts = torch.arange(0, E, call, device="cuda")
+    out = {"offsets": empty(N + 1, torch.int64), "ids": empty(2 * E, torch.int32),
+           "times": empty(2 * E, torch.float64), "eids": empty(2 * E, torch.int64)}
+    ws = empty(int(L.tgx_csr_build_workspace_size(2 * E)), torch.uint8)
+    a = _lib.TgxCsrBuildArgs(num_nodes=N, num_entries=2 * E, from_=src.data_ptr(), to=dst.data_ptr(),
+                             time=time.data_ptr(), call_starts=starts.data_ptr(), num_calls=starts.numel(),
+                             feat_dim=0, feat_dtype=_lib.TGX_F32, workspace=ws.data_ptr(), workspace_bytes=ws.numel(),
+                             flags=_lib.TGX_CSR_EVENTS_BY_CALL | flags,
+                             **{f"out_{k}": v.data_ptr() for k, v in out.items()})
+
+    def build(keep=(src, dst, time, starts, ws)):
+        _lib.check(L.tgx_csr_build(ctypes.byref(a), torch.cuda.current_stream().cuda_stream), "tgx_csr_build")
+
+    return build, out
+
+
+def test_build_order_is_a_permutation_while_times_change():
+    """The build order of runs of equal times takes every event twice even where another
+    stream writes the times while the build reads them: no position of the permutation
+    is left unwritten for the row gather to follow."""
+    E, N = 300_000, 1_000
+    src, dst = (torch.randint(0, N, (E,), device="cuda") for _ in range(2))
+    pair = [torch.full((E,), 3.0, dtype=torch.float64, device="cuda"),
+            torch.arange(E, dtype=torch.float64, device="cuda")]
+    time = pair[0].clone()
+    build, out = _by_call(N, src, dst, time, 10_000, _lib.TGX_CSR_NONDECREASING)
+    want = torch.arange(E, device="cuda").repeat_interleave(2)
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(20):
+        with torch.cuda.stream(other):
+            for i in range(8):
+                time.copy_(pair[i & 1])
+        build()
+        torch.cuda.synchronize()
+        assert torch.equal(out["eids"].sort().values, want)

@@ -157,12 +157,13 @@ __global__ __launch_bounds__(kThreads) void csr_scan_final(const ScanPart* __res
 // [2s, 2e) -- from->to of event k at s + k, then to->from at e + k -- which for
 // runs of a non-decreasing stream is already its stable time order.
 //
-// Two launches over tiles of kSegTile events.  Both mark the tile's segment
-// starts in an LDS bitmap (the same marks from the same inputs, so the segments
-// partition the events whatever the call starts hold): csr_seg_tiles writes each
-// tile's first and last start; csr_seg_order finds the starts nearest to its tile
-// from those, then each event's own segment from the bitmap, and writes the
-// entries at their positions.  8M events in runs of three take 13 + 91 us, the keys
+// Two launches over tiles of kSegTile events.  csr_seg_tiles marks the tile's
+// segment starts in a bitmap and writes that and the tile's first and last start;
+// csr_seg_order finds the starts nearest to its tile from those, then each event's
+// own segment from the bitmap, and writes the entries at their positions.  Times
+// and call starts are read for the marks once: the segments partition the events,
+// and the positions are a permutation, whatever the arrays hold, also where
+// another stream writes them meanwhile.  8M events in runs of three take 13 + 91 us, the keys
 // and records of the next steps included (448 MB; before, marks, a device-wide scan
 // of them, segment starts, the order and the node keys took eight launches and 230 us).
 constexpr int kSegItems = 8;
@@ -171,11 +172,14 @@ constexpr int kSegWords = kSegTile / 32;
 static_assert(kSegWords == kWave, "one bitmap word per lane");
 constexpr uint32_t kNoStart = 0xffffffffu;
 
-// bits[] = segment starts of events [base, base + kSegTile) (workgroup-wide; ends
-// with a barrier)
-__device__ __forceinline__ void seg_marks(const double* __restrict__ time, int64_t E, int runs,
-                                          const int64_t* __restrict__ starts, int64_t m, int64_t base,
-                                          uint32_t* bits) {
+// bitmap[tile][.] = the tile's segment starts; first[tile], last[tile]: its first and
+// last one (kNoStart: none)
+__global__ __launch_bounds__(kThreads) void csr_seg_tiles(const double* __restrict__ time, int64_t E, int runs,
+                                                          const int64_t* __restrict__ starts, int64_t m,
+                                                          uint32_t* __restrict__ bitmap, uint32_t* __restrict__ first,
+                                                          uint32_t* __restrict__ last) {
+  __shared__ uint32_t bits[kSegWords];
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kSegTile;
   if (threadIdx.x < kSegWords) bits[threadIdx.x] = 0u;
   // first call start at or after base, by 64-ary rounds of every wave
   const int lane = threadIdx.x & (kWave - 1);
@@ -208,17 +212,9 @@ __device__ __forceinline__ void seg_marks(const double* __restrict__ time, int64
     }
   }
   __syncthreads();
-}
-
-// first[tile], last[tile]: the tile's first and last segment start (kNoStart: none)
-__global__ __launch_bounds__(kThreads) void csr_seg_tiles(const double* __restrict__ time, int64_t E, int runs,
-                                                          const int64_t* __restrict__ starts, int64_t m,
-                                                          uint32_t* __restrict__ first, uint32_t* __restrict__ last) {
-  __shared__ uint32_t bits[kSegWords];
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kSegTile;
-  seg_marks(time, E, runs, starts, m, base, bits);
   if (threadIdx.x < kWave) {
     const uint32_t w = bits[threadIdx.x];
+    bitmap[static_cast<int64_t>(blockIdx.x) * kSegWords + threadIdx.x] = w;
     const uint64_t any = __ballot(w != 0);
     if (any == 0) {
       if (threadIdx.x == 0) first[blockIdx.x] = last[blockIdx.x] = kNoStart;
@@ -260,7 +256,7 @@ __device__ __forceinline__ uint32_t node_key(int64_t u, int64_t N) {
 template <bool RUNS>
 __global__ __launch_bounds__(kThreads) void csr_seg_order(
     const double* __restrict__ time, const int64_t* __restrict__ from, const int64_t* __restrict__ to, int64_t E,
-    int64_t N, const int64_t* __restrict__ starts, int64_t m, const uint32_t* __restrict__ first,
+    int64_t N, const uint32_t* __restrict__ bitmap, const uint32_t* __restrict__ first,
     const uint32_t* __restrict__ last, uint32_t* __restrict__ idx, uint64_t* __restrict__ tkey,
     uint32_t* __restrict__ nkey, EventRec* __restrict__ rec, int32_t* __restrict__ status) {
   __shared__ uint32_t bits[kSegWords], prev[kSegWords], next[kSegWords], edge[2];
@@ -273,11 +269,12 @@ __global__ __launch_bounds__(kThreads) void csr_seg_order(
     const uint32_t x = nearest_start(first, blockIdx.x, gridDim.x, 1, static_cast<uint32_t>(E));
     if (threadIdx.x == kWave) edge[1] = x;
   }
-  seg_marks(time, E, RUNS ? 1 : 0, starts, m, base, bits);
+  __syncthreads();
   if (threadIdx.x < kWave) {
     // the last start before word `lane` and the first one after it
     const int lane = threadIdx.x;
-    const uint32_t w = bits[lane];
+    const uint32_t w = bitmap[static_cast<int64_t>(blockIdx.x) * kSegWords + lane];
+    bits[lane] = w;
     const uint32_t at = static_cast<uint32_t>(base) + lane * 32;
     const uint64_t any = __ballot(w != 0);
     const uint32_t wl = w != 0 ? at + 31 - __builtin_clz(w) : 0u;
@@ -546,17 +543,20 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
   const bool ident = pairs && !by_call;  // already in stable time order
   bool keyed = false;                    // node keys and records are done
   if (by_call) {
-    // the build order from the segments; each tile's starts in nk[1] (free until the first pass)
+    // the build order from the segments; the tiles' bitmaps in nk[1] (kSegWords per kSegTile
+    // events: its n words hold them), their first and last starts in tk[1] (both free until
+    // the first pass)
     const unsigned gt = static_cast<unsigned>(cdiv(ne, kSegTile));
-    uint32_t* first = nk[1];
-    uint32_t* last = nk[1] + gt;
+    uint32_t* bitmap = nk[1];
+    uint32_t* first = reinterpret_cast<uint32_t*>(tk[1]);
+    uint32_t* last = first + gt;
     hipLaunchKernelGGL(csr_seg_tiles, dim3(gt), dim3(kThreads), 0, stream, a->time, ne, runs, a->call_starts,
-                       a->num_calls, first, last);
+                       a->num_calls, bitmap, first, last);
     if ((rc = check_launch("csr_seg_tiles"))) return rc;
     auto order = [&](auto kernel) {
-      hipLaunchKernelGGL(kernel, dim3(gt), dim3(kThreads), 0, stream, a->time, a->from, a->to, ne, N, a->call_starts,
-                         a->num_calls, static_cast<const uint32_t*>(first), static_cast<const uint32_t*>(last), ix[0],
-                         tk[0], nk[0], rec, a->status);
+      hipLaunchKernelGGL(kernel, dim3(gt), dim3(kThreads), 0, stream, a->time, a->from, a->to, ne, N,
+                         static_cast<const uint32_t*>(bitmap), static_cast<const uint32_t*>(first),
+                         static_cast<const uint32_t*>(last), ix[0], tk[0], nk[0], rec, a->status);
     };
     if (runs)
       order(csr_seg_order<true>);
