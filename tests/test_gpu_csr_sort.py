@@ -108,3 +108,39 @@ def test_build_order_is_a_permutation_while_times_change():
         build()
         torch.cuda.synchronize()
         assert torch.equal(out["eids"].sort().values, want)
+
+
+def test_segments_across_steps_of_tiles():
+    """Runs of equal times within, across and longer than the 4,096 tiles (8.4M events)
+    that one step of the search for a tile's neighbouring starts takes."""
+    E = 8_500_000
+    rng = np.random.default_rng(5)
+    src, dst = rng.integers(0, 900, E), rng.integers(0, 900, E)
+    edges = [1, 2_047, 2_048, 2_500, 40_960, 3_000_001, 3_000_002, 8_388_600, 8_388_650, 8_499_999]
+    time = 4.0 + np.searchsorted(edges, np.arange(E), side="right").astype(np.float64)
+    assert _check(900, 1, [0, 6_000_000, E], src, dst, time)._csr_build_mode == "runs"
+
+
+def test_long_calls_cost_no_more_than_short_ones():
+    """The build order of 64M events given by one call takes the time of the same events
+    in calls of 10,000: the search for a tile's neighbouring starts is linear in the
+    tiles (one that walks them from every tile costs 1.5 ms more here)."""
+    E, N = 64_000_000, 1_000_000
+    src, dst = (torch.randint(0, N, (E,), device="cuda") for _ in range(2))
+    time = torch.arange(E, dtype=torch.float64, device="cuda")
+    time[1::2] -= 3.0
+    took = {}
+    for call in (E, 10_000):
+        build, out = _by_call(N, src, dst, time, call)
+        build()
+        best = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            build()
+            b.record()
+            b.synchronize()
+            best.append(a.elapsed_time(b))
+        took[call] = min(best)
+        del build, out
+    assert took[E] - took[10_000] < 0.7, took

@@ -157,10 +157,10 @@ __global__ __launch_bounds__(kThreads) void csr_scan_final(const ScanPart* __res
 // [2s, 2e) -- from->to of event k at s + k, then to->from at e + k -- which for
 // runs of a non-decreasing stream is already its stable time order.
 //
-// Two launches over tiles of kSegTile events.  csr_seg_tiles marks the tile's
+// Three launches over tiles of kSegTile events.  csr_seg_tiles marks the tile's
 // segment starts in a bitmap and writes that and the tile's first and last start;
-// csr_seg_order finds the starts nearest to its tile from those, then each event's
-// own segment from the bitmap, and writes the entries at their positions.  Times
+// csr_seg_edges finds the starts nearest to each tile from those; csr_seg_order each
+// event's own segment from the bitmap, and writes the entries at their positions.  Times
 // and call starts are read for the marks once: the segments partition the events,
 // and the positions are a permutation, whatever the arrays hold, also where
 // another stream writes them meanwhile.  8M events in runs of three take 13 + 91 us, the keys
@@ -226,18 +226,53 @@ __global__ __launch_bounds__(kThreads) void csr_seg_tiles(const double* __restri
   }
 }
 
-// the value nearest to tile `t` in direction `dir` (-1, 1) among v[0, nt) that is
-// not kNoStart, else `none`; one wavefront
-__device__ __forceinline__ uint32_t nearest_start(const uint32_t* __restrict__ v, int64_t t, int64_t nt, int dir,
-                                                  uint32_t none) {
+// prev[t]: the last segment start before tile t (0: event 0 starts one), next[t]: the
+// first one after it (E), from the tiles' first and last starts.  Workgroup 0 walks the
+// tiles forwards, workgroup 1 backwards, kEdgeItems consecutive ones per thread and step:
+// linear in the tiles, however long a segment is: 20 us for 64M events, 4 for 8M.  (When
+// every tile of csr_seg_order walked its neighbours for itself, 64 at a time, 64M events
+// in one call took it 1,924 us, 356 now; 8M in one run of equal times 106, 74 now.)
+constexpr int kEdgeThreads = 1024;
+constexpr int kEdgeItems = 4;
+__global__ __launch_bounds__(kEdgeThreads) void csr_seg_edges(const uint32_t* __restrict__ first,
+                                                              const uint32_t* __restrict__ last, int64_t nt, int64_t E,
+                                                              uint32_t* __restrict__ prev, uint32_t* __restrict__ next) {
+  __shared__ uint32_t wlast[kEdgeThreads / kWave];
+  const bool back = blockIdx.x != 0;
+  const uint32_t* v = back ? first : last;
+  uint32_t* out = back ? next : prev;
   const int lane = threadIdx.x & (kWave - 1);
-  for (int64_t i = t + dir; i >= 0 && i < nt; i += dir * kWave) {  // wave-uniform
-    const int64_t j = i + static_cast<int64_t>(dir) * lane;
-    const uint32_t x = j >= 0 && j < nt ? v[j] : kNoStart;
-    const uint64_t any = __ballot(x != kNoStart);
-    if (any != 0) return static_cast<uint32_t>(__shfl(static_cast<int>(x), __builtin_ctzll(any)));
+  const int wv = threadIdx.x / kWave;
+  uint32_t carry = back ? static_cast<uint32_t>(E) : 0u;  // the latest start of the steps before
+  for (int64_t t0 = 0; t0 < nt; t0 += kEdgeThreads * kEdgeItems) {  // workgroup-uniform
+    const int64_t t = t0 + static_cast<int64_t>(threadIdx.x) * kEdgeItems;
+    uint32_t x[kEdgeItems];
+    uint32_t mine = kNoStart;  // the thread's latest start
+#pragma unroll
+    for (int r = 0; r < kEdgeItems; ++r) {
+      x[r] = t + r < nt ? v[back ? nt - 1 - (t + r) : t + r] : kNoStart;
+      mine = x[r] != kNoStart ? x[r] : mine;
+    }
+    const uint64_t any = __ballot(mine != kNoStart);
+    const uint64_t lower = any & ((uint64_t(1) << lane) - 1);
+    const uint32_t before = __shfl(mine, lower != 0 ? 63 - __builtin_clzll(lower) : 0);
+    const uint32_t top = __shfl(mine, any != 0 ? 63 - __builtin_clzll(any) : 0);
+    if (lane == 0) wlast[wv] = any != 0 ? top : kNoStart;
+    __syncthreads();
+    uint32_t run = carry;
+    for (int w = 0; w < kEdgeThreads / kWave; ++w) {
+      const uint32_t y = wlast[w];
+      if (w < wv && y != kNoStart) run = y;
+      if (y != kNoStart) carry = y;
+    }
+    if (lower != 0) run = before;
+#pragma unroll
+    for (int r = 0; r < kEdgeItems; ++r) {
+      if (t + r < nt) out[back ? nt - 1 - (t + r) : t + r] = run;
+      if (x[r] != kNoStart) run = x[r];
+    }
+    __syncthreads();  // wlast has been read
   }
-  return none;
 }
 
 // event record of the row gather: time and both ends
@@ -256,20 +291,11 @@ __device__ __forceinline__ uint32_t node_key(int64_t u, int64_t N) {
 template <bool RUNS>
 __global__ __launch_bounds__(kThreads) void csr_seg_order(
     const double* __restrict__ time, const int64_t* __restrict__ from, const int64_t* __restrict__ to, int64_t E,
-    int64_t N, const uint32_t* __restrict__ bitmap, const uint32_t* __restrict__ first,
-    const uint32_t* __restrict__ last, uint32_t* __restrict__ idx, uint64_t* __restrict__ tkey,
+    int64_t N, const uint32_t* __restrict__ bitmap, const uint32_t* __restrict__ tile_prev,
+    const uint32_t* __restrict__ tile_next, uint32_t* __restrict__ idx, uint64_t* __restrict__ tkey,
     uint32_t* __restrict__ nkey, EventRec* __restrict__ rec, int32_t* __restrict__ status) {
-  __shared__ uint32_t bits[kSegWords], prev[kSegWords], next[kSegWords], edge[2];
+  __shared__ uint32_t bits[kSegWords], prev[kSegWords], next[kSegWords];
   const int64_t base = static_cast<int64_t>(blockIdx.x) * kSegTile;
-  // the starts around the tile: event 0 is always one, the end of the last segment is E
-  if (threadIdx.x < kWave) {
-    const uint32_t x = nearest_start(last, blockIdx.x, gridDim.x, -1, 0u);
-    if (threadIdx.x == 0) edge[0] = x;
-  } else if (threadIdx.x < 2 * kWave) {
-    const uint32_t x = nearest_start(first, blockIdx.x, gridDim.x, 1, static_cast<uint32_t>(E));
-    if (threadIdx.x == kWave) edge[1] = x;
-  }
-  __syncthreads();
   if (threadIdx.x < kWave) {
     // the last start before word `lane` and the first one after it
     const int lane = threadIdx.x;
@@ -283,8 +309,8 @@ __global__ __launch_bounds__(kThreads) void csr_seg_order(
     const uint64_t upper = lane == 63 ? 0 : any >> (lane + 1);
     const uint32_t pl = __shfl(wl, lower != 0 ? 63 - __builtin_clzll(lower) : 0);
     const uint32_t nf = __shfl(wf, upper != 0 ? lane + 1 + __builtin_ctzll(upper) : 0);
-    prev[lane] = lower != 0 ? pl : edge[0];
-    next[lane] = upper != 0 ? nf : edge[1];
+    prev[lane] = lower != 0 ? pl : tile_prev[blockIdx.x];
+    next[lane] = upper != 0 ? nf : tile_next[blockIdx.x];
   }
   __syncthreads();
   int bad = 0;
@@ -544,19 +570,24 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
   bool keyed = false;                    // node keys and records are done
   if (by_call) {
     // the build order from the segments; the tiles' bitmaps in nk[1] (kSegWords per kSegTile
-    // events: its n words hold them), their first and last starts in tk[1] (both free until
-    // the first pass)
+    // events: its n words hold them), their first and last starts and the nearest ones around
+    // them in tk[1] (both free until the first pass)
     const unsigned gt = static_cast<unsigned>(cdiv(ne, kSegTile));
     uint32_t* bitmap = nk[1];
     uint32_t* first = reinterpret_cast<uint32_t*>(tk[1]);
     uint32_t* last = first + gt;
+    uint32_t* prev = last + gt;
+    uint32_t* next = prev + gt;
     hipLaunchKernelGGL(csr_seg_tiles, dim3(gt), dim3(kThreads), 0, stream, a->time, ne, runs, a->call_starts,
                        a->num_calls, bitmap, first, last);
     if ((rc = check_launch("csr_seg_tiles"))) return rc;
+    hipLaunchKernelGGL(csr_seg_edges, dim3(2), dim3(kEdgeThreads), 0, stream, static_cast<const uint32_t*>(first),
+                       static_cast<const uint32_t*>(last), static_cast<int64_t>(gt), ne, prev, next);
+    if ((rc = check_launch("csr_seg_edges"))) return rc;
     auto order = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(gt), dim3(kThreads), 0, stream, a->time, a->from, a->to, ne, N,
-                         static_cast<const uint32_t*>(bitmap), static_cast<const uint32_t*>(first),
-                         static_cast<const uint32_t*>(last), ix[0], tk[0], nk[0], rec, a->status);
+                         static_cast<const uint32_t*>(bitmap), static_cast<const uint32_t*>(prev),
+                         static_cast<const uint32_t*>(next), ix[0], tk[0], nk[0], rec, a->status);
     };
     if (runs)
       order(csr_seg_order<true>);
