@@ -144,3 +144,26 @@ def test_long_calls_cost_no_more_than_short_ones():
         took[call] = min(best)
         del build, out
     assert took[E] - took[10_000] < 0.7, took
+
+
+def test_more_wide_rows_than_one_launch_gathers():
+    """16.8M entries with rows above 8 KB (one entry per workgroup) are more workgroups
+    than one launch may hold: every entry is written."""
+    E, N = 8_388_700, 50_000
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 170e9:
+        pytest.skip("the rows take 138 GB")
+    rng = np.random.default_rng(8)
+    src, dst = (torch.from_numpy(rng.integers(0, N, E)).cuda() for _ in range(2))
+    time = torch.arange(E, dtype=torch.float64, device="cuda")
+    got = TemporalGraph(N, edge_feat_dim=2052, device="cuda", track_edge_ids=True)
+    want = TemporalGraph(N, edge_feat_dim=1, device="cuda", track_edge_ids=True)
+    for g in (want, got):
+        g.advance(src, dst, time)
+        g.freeze_csr()
+    for name in ("_offsets", "_nbr_ids", "_nbr_times", "_nbr_eids"):
+        assert torch.equal(getattr(got, name), getattr(want, name)), name
+    for s in range(0, 2 * E, 1 << 20):
+        assert not got._nbr_feats[s:s + (1 << 20)].any()
+    del got, g
+    torch.cuda.empty_cache()

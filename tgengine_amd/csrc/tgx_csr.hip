@@ -408,6 +408,10 @@ constexpr int kGatherChunks = kThreads * kGatherDepth;  // chunks a workgroup ho
 constexpr int kGatherMost = 256;                        // entries per workgroup at most
 constexpr int kXcds = 8;
 constexpr int kGatherSlice = 64;  // tiles of neighbouring events given to one XCD
+// tiles per launch: a launch holds fewer than 2^32 threads, which 16.8M entries of rows
+// above 8 KB (one per workgroup) would reach in one
+constexpr int64_t kGatherTiles = int64_t(1) << 20;
+static_assert(kGatherTiles % (kXcds * kGatherSlice) == 0, "whole slices per launch");
 
 // key of tile i (`per` entries) of the gather: its first entry's event
 __global__ __launch_bounds__(kThreads) void csr_tile_keys(const uint32_t* __restrict__ perm, int64_t ntiles, int per,
@@ -420,11 +424,12 @@ template <int VEC>
 __global__ __launch_bounds__(kThreads) void csr_gather(
     const uint32_t* __restrict__ perm, int64_t n, const EventRec* __restrict__ rec, int pairs,
     const int64_t* __restrict__ event, int64_t num_events, const uint8_t* __restrict__ feats, int64_t row_bytes, int nch,
-    uint32_t nch_magic, int per, const uint32_t* __restrict__ order, int64_t ntiles, int32_t* __restrict__ out_ids, double* __restrict__ out_times,
-    int64_t* __restrict__ out_eids, uint8_t* __restrict__ out_feats, int32_t* __restrict__ status) {
+    uint32_t nch_magic, int per, const uint32_t* __restrict__ order, int64_t tile0, int64_t ntiles,
+    int32_t* __restrict__ out_ids, double* __restrict__ out_times, int64_t* __restrict__ out_eids,
+    uint8_t* __restrict__ out_feats, int32_t* __restrict__ status) {
   using V = typename RowChunk<VEC>::T;
   __shared__ int64_t row[kGatherMost];  // an entry's feature row, -1: zeros
-  int64_t tile = blockIdx.x;
+  int64_t tile = tile0 + blockIdx.x;
   if (order != nullptr) {  // launch-uniform
     const int64_t g = tile / (kXcds * kGatherSlice);
     const int r = static_cast<int>(tile - g * (kXcds * kGatherSlice));
@@ -653,11 +658,12 @@ extern "C" int tgx_csr_build(const tgx_csr_build_args* a, void* stream_) {
     gblocks = cdiv(ntiles, kXcds * kGatherSlice) * (kXcds * kGatherSlice);
   }
   auto gather = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(gblocks)), dim3(kThreads), 0, stream,
-                       static_cast<const uint32_t*>(perm_in), n, static_cast<const EventRec*>(rec), pairs, a->event,
-                       a->num_events, static_cast<const uint8_t*>(a->feats), row_bytes, static_cast<int>(nch), magic, per, order, ntiles,
-                       a->out_ids, a->out_times, a->out_eids, static_cast<uint8_t*>(fe ? a->out_feats : nullptr),
-                       a->status);
+    for (int64_t t0 = 0; t0 < gblocks; t0 += kGatherTiles)
+      hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(std::min(gblocks - t0, kGatherTiles))), dim3(kThreads), 0,
+                         stream, static_cast<const uint32_t*>(perm_in), n, static_cast<const EventRec*>(rec), pairs,
+                         a->event, a->num_events, static_cast<const uint8_t*>(a->feats), row_bytes,
+                         static_cast<int>(nch), magic, per, order, t0, ntiles, a->out_ids, a->out_times, a->out_eids,
+                         static_cast<uint8_t*>(fe ? a->out_feats : nullptr), a->status);
   };
   if (vec == 16)
     gather(csr_gather<16>);
