@@ -317,3 +317,60 @@ def test_ring_less_routing_boundaries():
                 assert np.array_equal(r.timestamps.cpu().numpy().view(np.int64), o.times.view(np.int64)), case
                 assert np.array_equal(r.mask.cpu().numpy(), o.mask), case
                 assert np.array_equal(r.edge_feats.cpu().numpy(), o.feats), case
+
+
+def _time_us(fn, calls=40):
+    fn()
+    best = []
+    for _ in range(6):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        for _ in range(calls):
+            fn()
+        b.record()
+        b.synchronize()
+        best.append(a.elapsed_time(b) / calls * 1e3)
+    return min(best)
+
+
+def test_queries_after_their_own_window_cost_the_same():
+    """A query after its node's last entry is answered by the first loads, also when the
+    graph holds later times of other nodes: it takes no longer than one after every
+    entry (a search before the loads took it a third longer here)."""
+    old, half, Q, K = 3_000, 1_500_000, 8_000, 10
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    ids = lambda hi, n: torch.randint(0, hi, (n,), generator=gen, device="cuda")  # noqa: E731
+    src, dst = (torch.cat([ids(old, half), old + ids(100_000, 500_000)]) for _ in range(2))
+    t = torch.arange(half + 500_000, dtype=torch.float64, device="cuda")
+    g = TemporalGraph(old + 100_000, edge_feat_dim=172, device="cuda")
+    g.advance(src, dst, t, torch.randn(t.numel(), 172, generator=gen, device="cuda"))
+    g.freeze_csr()
+    nodes = ids(old, Q)
+    later, between = (torch.full((Q,), x, dtype=torch.float64, device="cuda") for x in (3e6, half + 1000.0))
+    r, s = g.recent(nodes, later, K), g.recent(nodes, between, K)
+    assert torch.equal(r.neighbor_ids, s.neighbor_ids) and torch.equal(r.edge_feats, s.edge_feats)
+    assert bool(s.mask.all())
+    a, b = _time_us(lambda: g.recent(nodes, later, K)), _time_us(lambda: g.recent(nodes, between, K))
+    assert b < 1.15 * a, (a, b)
+
+
+@pytest.mark.parametrize("K,d", [(20, 4), (64, 172), (33, 3), (100, 4)])
+def test_event_endpoints_and_negatives_in_one_launch(K, d):
+    """Endpoints search their windows first and negatives load first, in one launch: with
+    times inside the windows, at their entries, after a node's last entry and after all
+    of them, over windows shorter and longer than K."""
+    N, b = 300, 900
+    rng, g, csr, tmax, fdt = _stream(90 + K, N, d, False, E=12000)
+    src, t = _queries(rng, N, b, tmax)
+    dst, neg = _queries(rng, N, b, tmax)[0], _queries(rng, N, 2 * b, tmax)[0].reshape(b, 2)
+    for Q in (b, 60):
+        spec = GatherSpec(neighbors=NeighborSpec(k=K))
+        pb = DataPipeline(spec, g).prepare(RawBatch(src=cu(src[:Q]), dst=cu(dst[:Q]), time=cu(t[:Q]),
+                                                    neg=cu(neg[:Q])))
+        for got, nodes, qt in ((pb.src_neighbors, src[:Q], t[:Q]), (pb.dst_neighbors, dst[:Q], t[:Q]),
+                               (pb.neg_neighbors, neg[:Q].reshape(-1), np.repeat(t[:Q], 2))):
+            o = O.recent(nodes, qt, K, csr, None, d, fdt)
+            assert np.array_equal(got.neighbor_ids.cpu().numpy(), o.ids)
+            assert np.array_equal(got.timestamps.cpu().numpy().view(np.int64), o.times.view(np.int64))
+            assert np.array_equal(got.mask.cpu().numpy(), o.mask)
+            assert np.array_equal(got.edge_feats.cpu().numpy(), o.feats)

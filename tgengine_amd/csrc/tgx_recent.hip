@@ -84,7 +84,7 @@ struct Params {
   int ngroups;
   const void* gn[TGX_MAX_QUERY_GROUPS];
   const uint8_t* gv[TGX_MAX_QUERY_GROUPS];  // per-query validity or null
-  int gi32[TGX_MAX_QUERY_GROUPS];           // int32 node ids
+  int gflags[TGX_MAX_QUERY_GROUPS];         // kGroupI32, kGroupInside
   const double* gt[TGX_MAX_QUERY_GROUPS];
   int64_t goff[TGX_MAX_QUERY_GROUPS + 1];
   int gdiv[TGX_MAX_QUERY_GROUPS];
@@ -206,6 +206,9 @@ constexpr int kSplitGroupWaves = 4;
 // csr_split: rows of at least this many bytes stream, and the encodings beside
 // them go out as nontemporal stores
 constexpr int64_t kNtRowBytes = 64;
+// query group flags: int32 node ids; queries inside their nodes' windows (a steer)
+constexpr int kGroupI32 = 1;
+constexpr int kGroupInside = 2;
 // node ids per thread and step of the ring plan's batch scan when the plan runs
 // in a gather launch (its registers stay within the gather's)
 constexpr int kFusedPlanScan = 4;
@@ -311,8 +314,9 @@ __device__ __forceinline__ int64_t query_of(const Params& P, int64_t g, int j) {
 // chosen with compares against the group offsets (constant indices only, so the
 // arguments stay in registers)
 __device__ __forceinline__ void query_load(const Params& P, int64_t q, int64_t& node, double& qt,
-                                           bool& valid) {
+                                           bool& valid, bool& inside) {
   valid = true;
+  inside = false;
   if (P.ngroups == 0) {
     node = P.nodes[q];
     qt = P.qtimes[q];
@@ -323,7 +327,7 @@ __device__ __forceinline__ void query_load(const Params& P, int64_t q, int64_t& 
   const uint8_t* vp = P.gv[0];
   int64_t off = 0;
   int div = P.gdiv[0];
-  int i32 = P.gi32[0];
+  int flags = P.gflags[0];
 #pragma unroll
   for (int g = 1; g < TGX_MAX_QUERY_GROUPS; ++g) {
     if (g < P.ngroups && q >= P.goff[g]) {
@@ -332,11 +336,12 @@ __device__ __forceinline__ void query_load(const Params& P, int64_t q, int64_t& 
       vp = P.gv[g];
       off = P.goff[g];
       div = P.gdiv[g];
-      i32 = P.gi32[g];
+      flags = P.gflags[g];
     }
   }
   const int64_t l = q - off;
-  node = i32 ? static_cast<int64_t>(static_cast<const int32_t*>(np)[l]) : static_cast<const int64_t*>(np)[l];
+  inside = (flags & kGroupInside) != 0;
+  node = (flags & kGroupI32) != 0 ? static_cast<int64_t>(static_cast<const int32_t*>(np)[l]) : static_cast<const int64_t*>(np)[l];
   qt = tp[div == 1 ? l : static_cast<int64_t>(static_cast<uint32_t>(l) / static_cast<uint32_t>(div))];
   if (vp != nullptr) valid = vp[l] != 0;
 }
@@ -344,8 +349,8 @@ __device__ __forceinline__ void query_load(const Params& P, int64_t q, int64_t& 
 __device__ __forceinline__ int64_t query_node(const Params& P, int64_t q) {
   int64_t node;
   double qt;
-  bool valid;
-  query_load(P, q, node, qt, valid);
+  bool valid, inside;
+  query_load(P, q, node, qt, valid, inside);
   return node;
 }
 
@@ -582,8 +587,8 @@ void recent_fused(Params P) {
   }
   int64_t node = -1;
   double qt = 0.0;
-  bool qvalid = true;
-  if (q >= 0) query_load(P, q, node, qt, qvalid);
+  bool qvalid = true, inside = false;
+  if (q >= 0) query_load(P, q, node, qt, qvalid, inside);
   const bool bad = q >= 0 && qvalid && node >= P.N;
   if (bad && sl == 0 && part == 0 && P.status != nullptr) atomicAdd(&P.status[TGX_ST_BAD_QUERY_NODE], 1);
   const int64_t ur = node < 0 ? 0 : node;
@@ -981,12 +986,16 @@ void recent_fused(Params P) {
 // window then holds none), those entries are the answer, as the search would
 // find: three dependent round trips (query, offsets, entries) before the
 // stores, against five for recent_fused's search, staging and row copy.
-// A query that may fall inside its window (a time not after the CSR's largest one,
-// max_time, when that is finite) sends the search's first Bp-ary round in place of
-// those loads, and its entries once the search is done: loading them both ways cost
-// the entries' bytes again (12,000 queries inside their windows 13.5 -> 12.8 us; two
-// hops of 4,000 x 20, whose hop-2 queries all are, 45.3 -> 43.4 us).
-template <int NREG>
+// A window of at most K entries is in the lanes then, and its search with it; a longer
+// one's first Bp-ary search round goes out beside the loads when the query may be
+// inside (a time not after the CSR's largest one, max_time).
+// INSIDE: queries expected inside their windows (kGroupInside) send that round in place
+// of the loads, and load their entries once the search is done: both ways cost the
+// entries' bytes again (two hops of 4,000 x 20, whose hop-2 queries all are inside,
+// 45.2 -> 43.3 us).  Not so for any query that may be: those after their own windows,
+// which only the load can tell, would wait a round trip longer (4,000 of them over
+// windows of 60 entries, K = 20: 5.1 -> 5.6 us).
+template <int NREG, bool INSIDE>
 __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
   using VT = u32x4;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -1017,8 +1026,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
   if (q >= P.Q) q = -1;
   int64_t node = -1;
   double qt = 0.0;
-  bool qvalid = true;
-  if (q >= 0) query_load(P, q, node, qt, qvalid);
+  bool qvalid = true, inside = false;
+  if (q >= 0) query_load(P, q, node, qt, qvalid, inside);
   const bool bad = q >= 0 && qvalid && node >= P.N;
   if (bad && sl == 0 && P.status != nullptr) atomicAdd(&P.status[TGX_ST_BAD_QUERY_NODE], 1);
   // a padding node (< 0) has an empty window
@@ -1047,14 +1056,14 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
         if (k < P.nch) rows[k] = src[k];
     }
   };
-  // A query that may be inside its window (not after the CSR's largest time, when
-  // that is known) probes instead of loading entries it would throw away: the
-  // search's first Bp-ary round, probe sl at s0 + (sl + 1) step - 1, clamped to
-  // the last entry, so the top lane reads the window's last time.
+  // the search's first Bp-ary round, in place of the entries or beside them: probe sl
+  // at s0 + (sl + 1) step - 1, clamped to the last entry, so the top lane reads the
+  // window's last time
   const int Bp = 1 << lg;
   const int64_t wlen = s1 - s0;
-  const bool probing = wlen > 0 && qt <= P.c_tmax && P.c_tmax < __builtin_huge_val();
-  bool have = live && sl < K && s1 - K + sl >= s0 && !probing;
+  const bool first = INSIDE && inside && wlen > 0 && qt <= P.c_tmax && P.c_tmax < __builtin_huge_val();
+  const bool probing = first || (wlen > K && qt <= P.c_tmax);
+  bool have = live && sl < K && s1 - K + sl >= s0 && !first;
   if (have) load_entry(s1 - K + sl);
   const int64_t step = probing ? (wlen + Bp - 1) >> lg : 0;
   double tp = 0.0;
@@ -1063,18 +1072,21 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
     tp = P.c_times[pos < s1 ? pos : s1 - 1];
   }
   // sub-group uniform: lane K - 1 holds entry s1 - 1 whenever the window is not empty
-  const double tl = __shfl(probing ? tp : t, (h << lg) + (probing ? Bp : K) - 1);
+  const double tl = __shfl(first ? tp : t, (h << lg) + (first ? Bp : K) - 1);
   const bool after = !live || s1 == s0 || tl < qt;
 
   // ---- otherwise: search the window, then load the answer's entries ----
-  const uint64_t slow = __ballot(!after || probing);
+  const uint64_t slow = __ballot(!after || first);
   if (slow != 0) {  // wave-uniform
-    // the lower bound lies in [lo, hi]: after the first round, between the last
-    // probe below the query time and the next one
-    const uint64_t below = __ballot(probing && tp < qt) >> (h << lg);
+    // the lower bound lies in [lo, hi]: of a window in the lanes, behind its entries
+    // below the query time; after a first round, between the last probe below the
+    // query time and the next one
+    const uint64_t below = __ballot(probing ? tp < qt : have && t < qt) >> (h << lg);
+    const int64_t c = __popcll(Bp == kWave ? below : below & ((uint64_t(1) << Bp) - 1));
     int64_t lo = s0, hi = s1;
-    if (probing) {
-      const int64_t c = __popcll(Bp == kWave ? below : below & ((uint64_t(1) << Bp) - 1));
+    if (wlen <= K && !first) {
+      lo = hi = s0 + c;
+    } else if (probing) {
       const int64_t nl = s0 + c * step;
       const int64_t pc = s0 + (c + 1) * step - 1;
       lo = nl < s1 ? nl : s1;
@@ -1083,7 +1095,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
     // every sub-group searches its own query at once (Bp-ary rounds; one query
     // after another with 64-ary rounds took 2 x 3 rounds for C3's hop-2 windows)
     const int64_t end = subgroup_lower_bound(P.c_times, lo, hi, qt, !after, sl, h, lg);
-    if (!after || probing) {
+    if (!after || first) {
       const int64_t cnt = (after ? s1 : end) - s0;
       const int take = static_cast<int>(cnt < K ? cnt : K);
       have = sl < K && sl >= K - take;
@@ -1145,11 +1157,15 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_window(Params P) {
 // window's last time and the first kCopyDepth chunks per lane of its share of
 // their rows; when the query comes after its whole window those are the answer
 // (query, offsets, entries and first row chunks: three dependent round trips
-// before the first store, against five in recent_fused's ring-less copy).  A query
-// that may be inside its window searches first and then loads, as in csr_window:
-// 200 training events of a frozen Reddit-sized graph (K = 64, 688-byte rows) threw
-// away 20 MB of rows and took 17.4 us, 16.1 now.
-template <int VEC, bool RANGES>
+// before the first store, against five in recent_fused's ring-less copy).  INSIDE, as
+// in csr_window, for the endpoints of events: 200 training events of a frozen
+// Reddit-sized graph (K = 64, 688-byte rows) threw away 20 MB of rows and took 18.2 us,
+// 17.2 now.  Their negatives, one in three, load first: searching first took 16.7 us
+// there, but where 4,000 queries come after windows of 1,000 entries 15.6 instead of
+// 11.5 (K = 10).  With ranges every query loads first: where the encodings are the bulk
+// the queries that start late end late (LastFM's shape 27.1 us, with endpoints that
+// search first 27.9).
+template <int VEC, bool RANGES, bool INSIDE>
 __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   using VT = typename RowChunk<VEC>::T;
   extern __shared__ __align__(16) uint8_t smem[];
@@ -1190,8 +1206,8 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   if (q >= P.Q) q = -1;
   int64_t node = -1;
   double qt = 0.0;
-  bool qvalid = true;
-  if (q >= 0) query_load(P, q, node, qt, qvalid);
+  bool qvalid = true, inside = false;
+  if (q >= 0) query_load(P, q, node, qt, qvalid, inside);
   const bool bad = q >= 0 && qvalid && node >= P.N;
   if (bad && lane == 0 && part == 0 && P.status != nullptr) atomicAdd(&P.status[TGX_ST_BAD_QUERY_NODE], 1);
   // wave-uniform; a padding node (< 0) has an empty window
@@ -1212,11 +1228,10 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
     id = P.c_ids[x];
     if (P.o_eids != nullptr) eid = P.c_eids != nullptr ? P.c_eids[x] : -1;
   };
-  // A query that may be inside its window (not after the CSR's largest time, when
-  // that is known) does not load what it would throw away, but sends the search's
-  // first 64-ary round instead, clamped to the window's last entry.
-  const bool probing = s1 > s0 && qt <= P.c_tmax && P.c_tmax < __builtin_huge_val();  // wave-uniform
-  bool have = live && lane < np && s1 - K + pos >= s0 && !probing;
+  // INSIDE: the search's first 64-ary round in place of those loads, clamped to the
+  // window's last entry
+  const bool first = INSIDE && inside && s1 > s0 && qt <= P.c_tmax && P.c_tmax < __builtin_huge_val();  // wave-uniform
+  bool have = live && lane < np && s1 - K + pos >= s0 && !first;
   if (have) load_entry(s1 - K + pos);
   const bool fe = P.o_feats != nullptr && P.row_bytes > 0;
   const int nch = P.nch;
@@ -1228,7 +1243,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   for (int u = 0; u < kCopyDepth; ++u) v[u] = VT{};
   bool after = !live || s1 == s0;
   int64_t lo = s0, hi = s1;
-  if (probing) {
+  if (first) {
     const int64_t step = (s1 - s0 + kWave - 1) / kWave;
     const int64_t at = s0 + (lane + 1) * step - 1;
     const double tp = P.c_times[at < s1 ? at : s1 - 1];
@@ -1252,11 +1267,13 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
     }
     if (!RANGES) tl = __shfl(t, K - 1);  // entry s1 - 1 whenever the window is not empty
     after = after || tl < qt;
+    // without ranges a window of at most K entries is all in the lanes
+    if (!RANGES && !after && s1 - s0 <= K) lo = hi = s0 + __popcll(__ballot(have && t < qt));
   }
   // position p >= K - take holds entry base + p
   int64_t base = s1 - K;
   int take = live ? static_cast<int>(s1 - s0 < K ? s1 - s0 : K) : 0;
-  const bool reload = !after || probing;  // wave-uniform
+  const bool reload = !after || first;  // wave-uniform
   if (reload) {
     if (!after) {
       const int64_t cnt = wave_lower_bound<true>(P.c_times, lo, hi, qt, lane) - s0;
@@ -1521,6 +1538,7 @@ struct Launch {
   bool window = false;  // csr_window runs the launch
   bool csr_split = false;  // csr_split runs it
   bool csr_ranges = false;  // in position ranges (K above 64)
+  bool inside = false;  // some queries are expected inside their windows
   bool co_after = false;  // co_occurrence_events counts after the gather, with co
   Params co;
 };
@@ -1646,7 +1664,7 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
         return fail(TGX_ERR_ARG, "tgx_recent: bad query group %d", g);
       P.gn[g] = qg.nodes;
       P.gv[g] = qg.valid;
-      P.gi32[g] = (qg.flags & TGX_QG_NODES_I32) != 0;
+      P.gflags[g] = (qg.flags & TGX_QG_NODES_I32) != 0 ? kGroupI32 : 0;
       P.gt[g] = qg.times;
       P.gdiv[g] = qg.times_per;
       P.goff[g] = off;
@@ -1659,6 +1677,19 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
                     (long long)(a->num_groups * qg.times_per));
     }
     for (int g = a->num_query_groups; g <= TGX_MAX_QUERY_GROUPS; ++g) P.goff[g] = off;
+    // Queries that a ring-less gather expects inside their nodes' windows when their
+    // time is not after the CSR's largest: two-hop queries (the groups with a validity
+    // array), since the hop-1 entry they follow is in their node's window at that very
+    // time; and the endpoints of events (two leading groups at the same times), which a
+    // graph that already holds times after them has been given as a rule.  Others, such
+    // as negatives, may as well come after a node's last entry.
+    for (int g = 0; g < a->num_query_groups; ++g)
+      if (P.gv[g] != nullptr) P.gflags[g] |= kGroupInside;
+    if (a->num_query_groups >= 2 && P.gt[0] == P.gt[1] && P.gdiv[0] == 1 && P.gdiv[1] == 1) {
+      P.gflags[0] |= kGroupInside;
+      P.gflags[1] |= kGroupInside;
+    }
+    for (int g = 0; g < a->num_query_groups; ++g) L.inside |= (P.gflags[g] & kGroupInside) != 0;
     if (a->num_query_groups > 0 && off != a->num_queries)
       return fail(TGX_ERR_ARG, "tgx_recent: query groups hold %lld queries, num_queries is %lld",
                   (long long)off, (long long)a->num_queries);
@@ -1981,32 +2012,30 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
   pick(recent_fused<V, R, true, false>, recent_fused<V, R, false, false>, recent_fused<V, R, true, true>, \
        recent_fused<V, R, false, true>)
   if (L.window) {
+    auto window = [&](auto any, auto some) { L.inside ? launch(some) : launch(any); };
     if (L.nreg == 2)
-      launch(csr_window<2>);
+      window(csr_window<2, false>, csr_window<2, true>);
     else if (L.nreg == 4)
-      launch(csr_window<4>);
+      window(csr_window<4, false>, csr_window<4, true>);
     else
-      launch(csr_window<0>);
+      window(csr_window<0, false>, csr_window<0, true>);
   } else if (L.csr_split) {
-    if (L.csr_ranges) {
-      if (L.vec == 16)
-        launch(csr_split<16, true>);
-      else if (L.vec == kAnyRow)
-        launch(csr_split<kAnyRow, true>);
-      else if (L.vec == 4)
-        launch(csr_split<4, true>);
+    auto split = [&](auto any, auto some, auto ranges) {
+      if (L.csr_ranges)
+        launch(ranges);
       else
-        launch(csr_split<2, true>);
-    } else {
-      if (L.vec == 16)
-        launch(csr_split<16, false>);
-      else if (L.vec == kAnyRow)
-        launch(csr_split<kAnyRow, false>);
-      else if (L.vec == 4)
-        launch(csr_split<4, false>);
-      else
-        launch(csr_split<2, false>);
-    }
+        L.inside ? launch(some) : launch(any);
+    };
+#define TGX_SPLIT(V) split(csr_split<V, false, false>, csr_split<V, false, true>, csr_split<V, true, false>)
+    if (L.vec == 16)
+      TGX_SPLIT(16);
+    else if (L.vec == kAnyRow)
+      TGX_SPLIT(kAnyRow);
+    else if (L.vec == 4)
+      TGX_SPLIT(4);
+    else
+      TGX_SPLIT(2);
+#undef TGX_SPLIT
   } else if (L.vec == 16) {
     if (L.nreg == 2)
       TGX_PICK(16, 2);
