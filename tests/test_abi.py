@@ -198,6 +198,34 @@ def test_launch_shapes_stay_within_the_kernel_bounds():
     assert rc == 0 and sh[1] == 512 and sh[4] == 8 and sh[0] == 1  # with a ring: one workgroup
 
 
+def _event_args(k, b, csr, **more):
+    """Event-major (src, dst) queries of b events over a CSR alone, with co-occurrence."""
+    a = _lib.TgxRecentArgs(k=k, group=2, num_queries=2 * b, num_groups=b, num_query_groups=2,
+                           plan_mode=_lib.TGX_PLAN_EVENTS, out_ids=8, out_times=8, out_mask=8,
+                           co_mode=_lib.TGX_CO_FREQ, co_a=8, co_c=8, **more)
+    for g in range(2):
+        a.query_groups[g].nodes = 8
+        a.query_groups[g].times = 8
+        a.query_groups[g].count = b
+        a.query_groups[g].times_per = 1
+    return a
+
+
+def test_launches_hold_fewer_than_2_to_32_threads():
+    """A larger grid wraps around without an error: wide co-occurrence launches keep to the
+    kernel whose grid fits, and a launch that no kernel takes in one grid is refused."""
+    csr = _lib.TgxCsr(num_nodes=10, num_entries=5, feat_dim=0, feat_dtype=0, offsets=8, ids=8, times=8)
+    for k in (65, 129, 512):
+        for b in (200, 4_194_303, 4_194_304, 16_000_000):
+            rc, sh = _shape(None, ctypes.byref(csr), _event_args(k, b, csr))
+            assert rc == 0, _err()
+            assert sh[0] * sh[1] < 1 << 32, (k, b)
+            assert (sh[0] == b) == (b >= 4_194_304), (k, b)  # one workgroup per event
+    a = _lib.TgxRecentArgs(k=512, group=1, num_queries=9_000_000, nodes=8, times=8, out_ids=8, out_times=8, out_mask=8)
+    rc, _ = _shape(None, ctypes.byref(csr), a)
+    assert rc == 3 and "grid too large" in _err()
+
+
 def test_ring_less_launches_pack_queries_in_csr_window():
     """A CSR-only tiled launch of more than 2,048 queries at K <= 64 with rows of at
     most 64 bytes runs csr_window: 64 / Bp queries per wavefront (Bp = the power of

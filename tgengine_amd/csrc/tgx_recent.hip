@@ -182,6 +182,8 @@ __device__ __forceinline__ void put(T* p, const T& v) {
 
 // wavefronts per workgroup, the kernel's launch bound (512 threads)
 constexpr int kMaxWaves = 8;
+// threads of one launch (a larger grid wraps around, unreported)
+constexpr int64_t kLaunchThreads = int64_t(1) << 32;
 
 // queries of a launch above which small-row queries are packed several per wave
 // (about the wave slots of one MI355X: 256 CUs x 4 SIMDs x 8)
@@ -1755,10 +1757,12 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   // positions in LDS (10 KB at K = 512), which leaves two waves per query, where
   // csr_split runs eight (200 events at K = 512, 8-byte rows: 69.8 us in one launch,
   // 30.3 in two; at K <= 64 the one launch is the faster).  Timed launches
-  // (timing_start) stay one kernel.
+  // (timing_start) stay one kernel, and so do those of 8.4M queries or more: in
+  // csr_split they take up to kMaxWaves waves each, and a launch holds fewer than
+  // kLaunchThreads threads.
   if (mode == TGX_PLAN_EVENTS && ring == nullptr && P.has_csr && a->k > kWave && a->co_mode != TGX_CO_NONE &&
-      a->timing_start == nullptr && (reinterpret_cast<uintptr_t>(a->co_a) & 7) == 0 &&
-      (reinterpret_cast<uintptr_t>(a->co_c) & 7) == 0) {
+      a->num_queries < kLaunchThreads / (kMaxWaves * kWave) && a->timing_start == nullptr &&
+      (reinterpret_cast<uintptr_t>(a->co_a) & 7) == 0 && (reinterpret_cast<uintptr_t>(a->co_c) & 7) == 0) {
     L.co_after = true;
     L.co = P;
     mode = P.plan_mode = TGX_PLAN_TILES;
@@ -1934,8 +1938,9 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   P.plan_blocks = L.fuse_plan ? static_cast<int>((L.pl.n + kWave * waves - 1) / (kWave * waves)) : 0;
   L.lds = L.fuse_plan ? std::max(lds, plan_lds_bytes(kWave * waves)) : lds;
   L.blocks = nblocks + P.plan_blocks;
-  if (L.blocks >= (int64_t(1) << 31)) return fail(TGX_ERR_LIMIT, "tgx_recent: grid too large");
   L.threads = kWave * waves;
+  if (L.blocks >= (int64_t(1) << 31) || L.blocks * L.threads >= kLaunchThreads)
+    return fail(TGX_ERR_LIMIT, "tgx_recent: grid too large");
   L.qslots = qslots;
   L.vec = vec;
   L.nreg = nreg;
