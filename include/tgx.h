@@ -176,8 +176,10 @@ typedef struct tgx_recent_args {
   int32_t* status;         /* [TGX_STATUS_WORDS] or NULL */
   int32_t num_query_groups;                          /* 0 = use nodes/times */
   tgx_query_group query_groups[TGX_MAX_QUERY_GROUPS];
-  /* optional hipEvent_t pair recorded by the kernel dispatch itself (start and
-   * end of the kernel's execution); both NULL = plain launch */
+  /* optional hipEvent_t pair recorded by the dispatches themselves: the start of the
+   * gather kernel's execution and its end, or the end of the kernel that counts the
+   * pairs where that is a launch of its own (an event-major launch over a CSR alone
+   * with k above 64); the launches are the same as without.  Both NULL = plain launch */
   void* timing_start;
   void* timing_stop;
   /* optional ring plan run by the same launch (append_b > 0): tgx_ring_plan of

@@ -226,6 +226,15 @@ def test_launches_hold_fewer_than_2_to_32_threads():
     assert rc == 3 and "grid too large" in _err()
 
 
+def test_timed_launches_are_the_same_launches():
+    """timing_start / timing_stop change no kernel and no grid."""
+    csr = _lib.TgxCsr(num_nodes=10, num_entries=5, feat_dim=0, feat_dtype=0, offsets=8, ids=8, times=8)
+    for k in (20, 65, 512):
+        plain = _shape(None, ctypes.byref(csr), _event_args(k, 200, csr))
+        assert plain[0] == 0 and plain == _shape(None, ctypes.byref(csr), _event_args(k, 200, csr, timing_start=8,
+                                                                                     timing_stop=8))
+
+
 def test_ring_less_launches_pack_queries_in_csr_window():
     """A CSR-only tiled launch of more than 2,048 queries at K <= 64 with rows of at
     most 64 bytes runs csr_window: 64 / Bp queries per wavefront (Bp = the power of

@@ -1756,12 +1756,11 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   // counts its pairs afterwards: in the pair's workgroup every wave keeps all K
   // positions in LDS (10 KB at K = 512), which leaves two waves per query, where
   // csr_split runs eight (200 events at K = 512, 8-byte rows: 69.8 us in one launch,
-  // 30.3 in two; at K <= 64 the one launch is the faster).  Timed launches
-  // (timing_start) stay one kernel, and so do those of 8.4M queries or more: in
-  // csr_split they take up to kMaxWaves waves each, and a launch holds fewer than
-  // kLaunchThreads threads.
+  // 30.3 in two; at K <= 64 the one launch is the faster).  Launches of 8.4M queries
+  // or more stay one kernel: in csr_split they take up to kMaxWaves waves each, and a
+  // launch holds fewer than kLaunchThreads threads.
   if (mode == TGX_PLAN_EVENTS && ring == nullptr && P.has_csr && a->k > kWave && a->co_mode != TGX_CO_NONE &&
-      a->num_queries < kLaunchThreads / (kMaxWaves * kWave) && a->timing_start == nullptr &&
+      a->num_groups > 0 && a->num_queries < kLaunchThreads / (kMaxWaves * kWave) &&
       (reinterpret_cast<uintptr_t>(a->co_a) & 7) == 0 && (reinterpret_cast<uintptr_t>(a->co_c) & 7) == 0) {
     L.co_after = true;
     L.co = P;
@@ -1995,7 +1994,7 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
   const dim3 block(static_cast<unsigned>(L.threads));
   auto launch = [&](auto kernel) {
     if (ev0 != nullptr)
-      hipExtLaunchKernelGGL(kernel, grid, block, L.lds, stream, ev0, ev1, 0, L.P);
+      hipExtLaunchKernelGGL(kernel, grid, block, L.lds, stream, ev0, L.co_after ? nullptr : ev1, 0, L.P);
     else
       hipLaunchKernelGGL(kernel, grid, block, L.lds, stream, L.P);
   };
@@ -2057,8 +2056,12 @@ extern "C" int tgx_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_re
   }
 #undef TGX_PICK
   rc = check_launch(L.window ? "csr_window" : L.csr_split ? "csr_split" : "recent_fused");
-  if (rc == TGX_OK && L.co_after && L.co.ev_b > 0) {
-    hipLaunchKernelGGL(co_occurrence_events, dim3(static_cast<unsigned>(L.co.ev_b)), dim3(kCoThreads), 0, stream, L.co);
+  if (rc == TGX_OK && L.co_after) {
+    const dim3 pairs(static_cast<unsigned>(L.co.ev_b));
+    if (ev0 != nullptr)
+      hipExtLaunchKernelGGL(co_occurrence_events, pairs, dim3(kCoThreads), 0, stream, nullptr, ev1, 0, L.co);
+    else
+      hipLaunchKernelGGL(co_occurrence_events, pairs, dim3(kCoThreads), 0, stream, L.co);
     rc = check_launch("co_occurrence_events");
   }
   if (rc != TGX_OK || !L.want_plan || L.fuse_plan) return rc;
