@@ -178,7 +178,7 @@ typedef struct tgx_recent_args {
   tgx_query_group query_groups[TGX_MAX_QUERY_GROUPS];
   /* optional hipEvent_t pair recorded by the dispatches themselves: the start of the
    * gather kernel's execution and its end, or the end of the kernel that counts the
-   * pairs where that is a launch of its own (an event-major launch over a CSR alone
+   * pairs where that is a launch of its own (some event-major launches over a CSR alone
    * with k above 64); the launches are the same as without.  Both NULL = plain launch */
   void* timing_start;
   void* timing_stop;

@@ -215,7 +215,7 @@ def test_launches_hold_fewer_than_2_to_32_threads():
     """A larger grid wraps around without an error: wide co-occurrence launches keep to the
     kernel whose grid fits, and a launch that no kernel takes in one grid is refused."""
     csr = _lib.TgxCsr(num_nodes=10, num_entries=5, feat_dim=0, feat_dtype=0, offsets=8, ids=8, times=8)
-    for k in (65, 129, 512):
+    for k in (129, 200, 512):
         for b in (200, 4_194_303, 4_194_304, 16_000_000):
             rc, sh = _shape(None, ctypes.byref(csr), _event_args(k, b, csr))
             assert rc == 0, _err()
@@ -224,6 +224,24 @@ def test_launches_hold_fewer_than_2_to_32_threads():
     a = _lib.TgxRecentArgs(k=512, group=1, num_queries=9_000_000, nodes=8, times=8, out_ids=8, out_times=8, out_mask=8)
     rc, _ = _shape(None, ctypes.byref(csr), a)
     assert rc == 3 and "grid too large" in _err()
+
+
+def test_wide_co_occurrence_launches():
+    """Pairs are counted in a launch of their own (the gather then takes whole queries, not
+    events, per workgroup) above K = 128, for few queries, and for DyGFormer counts beside
+    short entries; K up to 128 otherwise keeps one launch, which streams wide entries better."""
+    csr = _lib.TgxCsr(num_nodes=10, num_entries=5, feat_dim=172, feat_dtype=0, offsets=8, ids=8, times=8, feats=16)
+    dyg = dict(co_mode=_lib.TGX_CO_DYGFORMER)
+    for k, b, d, more, one in ((100, 3000, 172, {}, True), (100, 3000, 172, dyg, True), (65, 129, 0, {}, True),
+                               (128, 200, 2, {}, True), (129, 200, 2, {}, False), (100, 128, 172, {}, False),
+                               (100, 3000, 2, dyg, False), (100, 3000, 64, dyg, False), (100, 3000, 65, dyg, True)):
+        csr.feat_dim = d
+        a = _event_args(k, b, csr, out_feats=16 if d else 0)
+        for name, v in more.items():
+            setattr(a, name, v)
+        rc, sh = _shape(None, ctypes.byref(csr), a)
+        assert rc == 0, _err()
+        assert (sh[0] == b) == one, (k, b, d, more)
 
 
 def test_timed_launches_are_the_same_launches():

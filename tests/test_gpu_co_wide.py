@@ -1,6 +1,7 @@
 """Co-occurrence of wide launches (K above 32) through DataPipeline.prepare against the
-oracle: over a frozen CSR alone (K above 64 counts in a launch of its own) and with a
-ring beside it (counted in the gather), both modes, with hubs, padding and pad nodes."""
+oracle: over a frozen CSR alone (K above 128, and above 64 for few queries, counts in a
+launch of its own) and with a ring beside it (counted in the gather), both modes, with
+hubs, padding and pad nodes."""
 import ctypes
 
 import numpy as np
@@ -17,7 +18,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("mode", ["freq", "dygformer"])
 @pytest.mark.parametrize("with_ring", [False, True])
-@pytest.mark.parametrize("K,n_neg", [(33, 1), (64, 3), (65, 1), (130, 7), (511, 1), (512, 2)])
+@pytest.mark.parametrize("K,n_neg", [(33, 1), (64, 3), (65, 1), (100, 9), (128, 11), (130, 7), (511, 1), (512, 2)])
 def test_wide_co_occurrence(K, n_neg, with_ring, mode):
     N = 30
     rng, g, csr, ring, tmax = _tied_graph(70 + K, N, 32, 2, 4, 700, 3 if with_ring else 0, 90)

@@ -208,6 +208,8 @@ constexpr int kSplitGroupWaves = 4;
 // csr_split: rows of at least this many bytes stream, and the encodings beside
 // them go out as nontemporal stores
 constexpr int64_t kNtRowBytes = 64;
+// co-occurrence counted in a launch of its own: entries (row and encoding) up to this many bytes
+constexpr int64_t kShortEntryBytes = 256;
 // query group flags: int32 node ids; queries inside their nodes' windows (a steer)
 constexpr int kGroupI32 = 1;
 constexpr int kGroupInside = 2;
@@ -1752,15 +1754,23 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   P.co_pair = a->co_pair;
   P.status = a->status;
 
-  // An event-major launch over a CSR alone with K above 64 gathers as csr_split and
-  // counts its pairs afterwards: in the pair's workgroup every wave keeps all K
+  // An event-major launch over a CSR alone with K above 64 may gather as csr_split and
+  // count its pairs afterwards: in the pair's workgroup every wave keeps all K
   // positions in LDS (10 KB at K = 512), which leaves two waves per query, where
   // csr_split runs eight (200 events at K = 512, 8-byte rows: 69.8 us in one launch,
-  // 30.3 in two; at K <= 64 the one launch is the faster).  Launches of 8.4M queries
-  // or more stay one kernel: in csr_split they take up to kMaxWaves waves each, and a
-  // launch holds fewer than kLaunchThreads threads.
+  // 30.3 in two).  It does so above K = 128 (at K = 200 two launches take 0.35 to 1.12
+  // of one's time over rows of 0 to 2,048 bytes and 20 to 3,000 events); up to there
+  // only where one launch would leave CUs idle (20 events at K = 100: 7.4 to 19 us
+  // against 7.9 to 29) or its K^2 counting is the bulk (the DyGFormer counts beside
+  // short entries: 0.7 to 0.9 of one's time), since wide entries stream better from
+  // one (1,000 events, K = 100, 688-byte rows and encodings: 94 us in two, 83 in one).
+  // Launches of 8.4M queries or more stay one kernel: in csr_split they take up to
+  // kMaxWaves waves each, and a launch holds fewer than kLaunchThreads threads.
+  const bool count_after =
+      a->k > 2 * kWave || a->num_queries <= kDeviceCUs ||
+      (a->co_mode == TGX_CO_DYGFORMER && P.row_bytes + 4 * a->d_t <= kShortEntryBytes);
   if (mode == TGX_PLAN_EVENTS && ring == nullptr && P.has_csr && a->k > kWave && a->co_mode != TGX_CO_NONE &&
-      a->num_groups > 0 && a->num_queries < kLaunchThreads / (kMaxWaves * kWave) &&
+      count_after && a->num_groups > 0 && a->num_queries < kLaunchThreads / (kMaxWaves * kWave) &&
       (reinterpret_cast<uintptr_t>(a->co_a) & 7) == 0 && (reinterpret_cast<uintptr_t>(a->co_c) & 7) == 0) {
     L.co_after = true;
     L.co = P;
