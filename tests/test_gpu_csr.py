@@ -115,7 +115,7 @@ def test_csr_build_empty():
 
 
 def test_csr_build_many_tiles_and_wide_node_ids():
-    # 2.4M entries (1,200 radix tiles), node ids over 21 bits (three node passes)
+    # 2.4M entries (586 radix tiles of 4,096), node ids over 21 bits (three node passes)
     rng = np.random.default_rng(12)
     N = 1_500_000
     batches = _batches(rng, N, [400_000, 800_000], 4, True, tie_grid=0.25)
@@ -123,9 +123,10 @@ def test_csr_build_many_tiles_and_wide_node_ids():
     _compare(g, ref)
 
 
-def test_csr_build_three_level_count_scan():
-    # 34M entries: 16,602 tiles x 256 digits = 4.25M counts > 2048^2, so the
-    # exclusive scan of the digit counts recurses twice
+def test_csr_build_one_large_out_of_order_call():
+    # 34M entries: 8,301 radix tiles over 1,024 ranges (nine tiles of 4,096 keys in most);
+    # 17M events of one call: 8,301 segment tiles with no start but the first event's,
+    # over three steps of the search for their neighbouring starts
     rng = np.random.default_rng(13)
     N, b = 100_000, 17_000_000
     src = rng.integers(0, N, b).astype(np.int64)

@@ -12,25 +12,30 @@ import torch
 from oracle import spec as O
 from tgengine_amd import TemporalGraph
 from tgengine_amd.core import _lib
+from tgengine_amd.synthetic import f32_to_bf16_bits
 
 pytestmark = pytest.mark.gpu
 
 
-def _check(N, d, cuts, src, dst, time, seed=0):
+def _check(N, d, cuts, src, dst, time, seed=0, bf16=False):
     E = len(src)
     feat = np.random.default_rng(seed).standard_normal((E, d)).astype(np.float32)
-    g = TemporalGraph(N, edge_feat_dim=d, device="cuda", track_edge_ids=True)
+    g = TemporalGraph(N, edge_feat_dim=d, device="cuda", track_edge_ids=True,
+                      feat_dtype=torch.bfloat16 if bf16 else torch.float32)
     events = []
     dev = [torch.from_numpy(x).cuda() for x in (src, dst, time, feat)]
+    if bf16:
+        feat = f32_to_bf16_bits(feat)
     for lo, hi in zip(cuts[:-1], cuts[1:]):
         g.advance(*(x[lo:hi] for x in dev))
         events.append((src[lo:hi], dst[lo:hi], time[lo:hi], feat[lo:hi], lo))
     g.freeze_csr()
-    ref = O.csr_freeze(N, d, events)
+    ref = O.csr_freeze(N, d, events, feat.dtype)
     assert np.array_equal(g._offsets.cpu().numpy(), ref.offsets)
     assert np.array_equal(g._nbr_ids.cpu().numpy(), ref.ids)
     assert np.array_equal(g._nbr_times.cpu().numpy().view(np.int64), ref.times.view(np.int64))
-    assert np.array_equal(g._nbr_feats.cpu().numpy(), ref.feats)
+    feats = g._nbr_feats.view(torch.int16).cpu().numpy().view(np.uint16) if bf16 else g._nbr_feats.cpu().numpy()
+    assert np.array_equal(feats, ref.feats)
     assert np.array_equal(g._nbr_eids.cpu().numpy(), ref.eids)
     assert g.status()["bad_event_nodes"] == 0
     return g
@@ -66,6 +71,16 @@ def test_sort_and_gather_sizes(E, N, d, order):
         time = time.reshape(-1, 100)[:, ::-1].reshape(-1).copy()
     g = _check(N, d, [0, E // 3, E], src, dst, time)
     assert g._csr_build_mode == {"strict": "pairs", "ties": "runs", "shuffled": "sort"}[order]
+
+
+# 256, 170, 93 and 64 entries per workgroup, the last one short, in rows of aligned and
+# of overlapping 16-byte chunks
+@pytest.mark.parametrize("d,bf16", [(5, False), (17, True), (22, False), (43, False), (64, False), (86, True)])
+def test_event_ordered_gather_widths(d, bf16):
+    E, N = 524_299, 3_000
+    rng = np.random.default_rng(d)
+    src = np.minimum((N * rng.random(E) ** 4).astype(np.int64), N - 1)
+    _check(N, d, [0, 200_001, E], src, rng.integers(0, N, E), 5.0 + np.arange(E, dtype=np.float64), bf16=bf16)
 
 
 def _by_call(N, src, dst, time, call, flags=0):
