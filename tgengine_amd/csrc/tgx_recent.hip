@@ -229,29 +229,18 @@ struct FastDiv {
   __device__ __forceinline__ uint32_t div(uint32_t x) const { return n > 1 ? __umulhi(x, m) : x; }
 };
 
-// smallest i in [lo, hi] with i == hi or t[i] >= q (t ascending); wave-uniform result
-template <bool CLAMP>
+// smallest i in [lo, hi] with i == hi or t[i] >= q (t ascending); wave-uniform result.
+// Probes are clamped to the window's last entry, so they stay in order and the top
+// lane reads t[hi - 1]: a query after the whole window ends in one round.
 __device__ __forceinline__ int64_t wave_lower_bound(const double* __restrict__ t, int64_t lo,
                                                     int64_t hi, double q, int lane) {
   while (hi - lo > kWave) {
     const int64_t step = (hi - lo + kWave - 1) / kWave;
     const int64_t pos0 = lo + static_cast<int64_t>(lane + 1) * step - 1;
-    int64_t pc, nl;
-    if constexpr (CLAMP) {
-      // probes clamped to the window's last entry, so they stay in order and the
-      // top lane reads t[hi - 1]: a query after the whole window ends in one round
-      const int64_t pos = pos0 < hi ? pos0 : hi - 1;
-      const int c = __popcll(__ballot(t[pos] < q));
-      pc = lo + static_cast<int64_t>(c + 1) * step - 1;
-      nl = lo + static_cast<int64_t>(c) * step;
-      nl = nl < hi ? nl : hi;  // every probe below q: lo = hi, and the search ends
-    } else {
-      const bool pr = pos0 < hi && t[pos0] < q;
-      const int c = __popcll(__ballot(pr));
-      pc = lo + static_cast<int64_t>(c + 1) * step - 1;
-      nl = lo + static_cast<int64_t>(c) * step;
-    }
-    lo = nl;
+    const int c = __popcll(__ballot(t[pos0 < hi ? pos0 : hi - 1] < q));
+    const int64_t pc = lo + static_cast<int64_t>(c + 1) * step - 1;
+    const int64_t nl = lo + static_cast<int64_t>(c) * step;
+    lo = nl < hi ? nl : hi;  // every probe below q: lo = hi, and the search ends
     hi = pc < hi ? pc : hi;
   }
   const int64_t pos = lo + lane;
@@ -259,7 +248,7 @@ __device__ __forceinline__ int64_t wave_lower_bound(const double* __restrict__ t
   return lo + __popcll(__ballot(pr));
 }
 
-// wave_lower_bound<true> run by every sub-group of Bp = 2^lg lanes at once on
+// wave_lower_bound run by every sub-group of Bp = 2^lg lanes at once on
 // its own query (lo, hi and q uniform within the sub-group h; active: whether
 // the sub-group searches at all): Bp-ary rounds with probes clamped to hi - 1,
 // until at most Bp entries are left.  Returns the first index in [lo, hi] whose
@@ -518,14 +507,15 @@ __device__ __forceinline__ void co_occurrence_pair(const Params& P, int64_t g, i
 // Waves-per-SIMD target: 8 for the ring-only event- and list-plan kernels with rows
 // through memory, whose bandwidth needs every resident wave (plan-group workgroups
 // of 6 waves fit 5 per CU at 8, 4 at 7; without the target C5's gather took 200 us
-// instead of 176); none for the tiled kernels of 16-byte chunks and the tiled CSR
-// copies, where forcing 8 capped the scalar registers and spilled them into their
-// own code (8.56 -> 7.74 us on C1 and 367 -> 356 us on C4 without it), nor for the
-// event-plan CSR copies with rows through memory; 7 for the rest, where it keeps a
-// private segment (a scalar spill's) out of the kernel.
+// instead of 176).  7 for those with rows in registers, which then spill up to 3
+// scalars instead of 20 and run 8 waves, and for the event-plan CSR copy of 2-byte
+// chunks (6,000 events, K = 64, 6-byte rows: 141 -> 131 us).  None for the other
+// event-plan CSR copies, whose 62 to 67 vector registers leave 7 waves, nor for the
+// tiled kernels, where a target spilled scalars into their own code (8 with 16-byte
+// chunks: 7.74 -> 8.56 us on C1, 356 -> 367 on C4; 7 with 4-byte chunks: 18,000
+// queries, K = 64, 12-byte rows 177 -> 184 us).
 template <int VEC, int NREG, bool TILES, bool CSR>
-constexpr int kWavesPerEu = TILES ? (VEC == 16 || VEC == kAnyRow || CSR ? 1 : 7)
-                                  : CSR ? (NREG > 0 || VEC == 2 ? 7 : 1) : (NREG > 0 ? 7 : 8);
+constexpr int kWavesPerEu = TILES ? 1 : NREG > 0 ? 7 : !CSR ? 8 : VEC == 2 ? 7 : 1;
 
 // TILES: the launch's plan mode is TGX_PLAN_TILES (no event or list plan, so no
 // co-occurrence); that copy of the kernel carries none of their code, which
@@ -1280,7 +1270,7 @@ __global__ __launch_bounds__(kMaxWaves * kWave) void csr_split(Params P) {
   const bool reload = !after || first;  // wave-uniform
   if (reload) {
     if (!after) {
-      const int64_t cnt = wave_lower_bound<true>(P.c_times, lo, hi, qt, lane) - s0;
+      const int64_t cnt = wave_lower_bound(P.c_times, lo, hi, qt, lane) - s0;
       take = static_cast<int>(cnt < K ? cnt : K);
       base = s0 + cnt - K;
     }
@@ -1820,8 +1810,8 @@ int setup_recent(const tgx_ring* ring, const tgx_csr* csr, const tgx_recent_args
   // holds at most kMaxWaves waves (the kernel's launch bound): its query slots
   // (the plan group, or `group` consecutive tiles) times split.
   const int qwant = mode != TGX_PLAN_TILES ? a->group : 1;
-  // waves whose LDS fits the CU's 160 KB next to the encoder weights (a large K
-  // with a CSR window takes about 24 KB per wave)
+  // waves whose LDS fits the CU's 160 KB next to the encoder weights (K = 512
+  // with a CSR window and a ring takes 17 KB per wave, 21 with edge ids)
   const int lds_waves = static_cast<int>((160 * 1024 - P.te_bytes) / P.wave_bytes);
   const int wave_cap = lds_waves < kMaxWaves ? lds_waves : kMaxWaves;
   // A launch whose workgroups all fit on the device at once at one wave per

@@ -25,14 +25,16 @@
 //   count  : tickets, in no particular order.
 //   groups : the ticket-0 entry of every node seen more than once reserves
 //            a contiguous list of c slots and a group id, small (c <= 64)
-//            or large (one atomic per wave, offsets by a wave scan).
+//            or large (three atomics per workgroup, offsets by wave scans).
 //   fill   : list[base[u] + ticket] = entry index.
 //   commit : singletons (c == 1) are written directly; a small group is ranked
-//            by one wavefront in registers, a large group by a whole workgroup
-//            over bitmap windows walked down from the top of the batch; the
-//            counters are restored to zero.
-// Every path writes the kept entries and advances write_pos.  Feature rows move
-// as 16-byte vectors when the row allows it.
+//            by one wavefront in registers, a large group by a whole workgroup:
+//            up to kCountedGroup entries by counting the later ones in LDS, a
+//            longer list over bitmap windows, each ending at the last entry not
+//            yet seen, until its kept entries are found; the counters are
+//            restored to zero.
+// Every path writes the kept entries and advances write_pos.  Feature rows of at
+// least 16 bytes move as 16-byte vectors (tgx_rows.h).
 #include "tgx_ring_plan.h"
 #include "tgx_rows.h"
 
@@ -41,8 +43,6 @@
 
 namespace tgx {
 namespace {
-
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
 constexpr int kCommitWaves = kThreads / kWave;
@@ -480,9 +480,7 @@ __global__ __launch_bounds__(kThreads) void append_commit(AppendParams P) {
     }
     return;
   }
-  // large groups (c > 64), one per workgroup, strided over the remaining blocks:
-  // the workgroup ranks the list over bitmap windows of kWinBits entry indices,
-  // from the top of the batch down, until `kept` entries are found
+  // large groups (c > 64), one per workgroup, strided over the remaining blocks
   const int64_t nlarge = P.ctl[kCtlLarge];
   const int64_t gstride = static_cast<int64_t>(gridDim.x) - P.ga - P.gb;
   for (int64_t gid = blk - P.ga - P.gb; gid < nlarge; gid += gstride)  // workgroup-uniform
