@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from tgengine_amd import TemporalGraph
+from tgengine_amd.core import temporal_graph
 
 pytestmark = pytest.mark.gpu
 
@@ -35,8 +36,10 @@ def _arrays(E, kind):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kind", ["plain", "host", "int32", "strided", "offset", "longer", "none"])
 @pytest.mark.parametrize("E", [1, 25_000])
-def test_from_dataset_equals_replay(E, kind, dtype):
+@pytest.mark.parametrize("copy", [0, 1 << 40])
+def test_from_dataset_equals_replay(E, kind, dtype, copy, monkeypatch):
     src, dst, time, feat = _arrays(E, kind)
+    monkeypatch.setattr(temporal_graph, "_ADOPT_COPY_BYTES", copy)
     g = TemporalGraph.from_dataset(src, dst, time, feat, 50, feat_dtype=dtype, track_edge_ids=True)
     r = TemporalGraph(50, edge_feat_dim=12 if feat is not None else 172, feat_dtype=dtype, track_edge_ids=True)
     for s in range(0, E, 10_000):
@@ -61,11 +64,14 @@ def test_from_dataset_refusals():
         TemporalGraph.from_dataset(src, dst, time, feat, 5)
 
 
+@pytest.mark.parametrize("copy", [False, True])
 @pytest.mark.parametrize("order", ["strict", "ties", "shuffled"])
-def test_from_dataset_leaves_its_arrays_to_other_streams(order):
-    """When from_dataset returns, nothing reads its arrays any more: a second stream
-    that never waits for the caller's refills them at once, and arrays allocated on a
-    loader's stream go back to that stream's pool and are handed out again."""
+def test_from_dataset_leaves_its_arrays_to_other_streams(order, copy, monkeypatch):
+    """When from_dataset returns, nothing reads its arrays any more, copied or read in
+    place: a second stream that never waits for the caller's refills them at once, and
+    arrays allocated on a loader's stream go back to that stream's pool and are handed
+    out again."""
+    monkeypatch.setattr(temporal_graph, "_ADOPT_COPY_BYTES", 1 << 40 if copy else 0)
     E, N, d = 400_000, 5_000, 64
     gen = torch.Generator(device="cuda").manual_seed(3)
     src = torch.randint(0, N, (E,), generator=gen, device="cuda")
@@ -83,7 +89,8 @@ def test_from_dataset_leaves_its_arrays_to_other_streams(order):
             arrays = [x.clone() for x in (src, dst, time, feat)]
         torch.cuda.current_stream().wait_stream(other)
         g = TemporalGraph.from_dataset(*arrays, N, track_edge_ids=True)
-        assert torch.cuda.current_stream().query()  # the build is over
+        if not copy:
+            assert torch.cuda.current_stream().query()  # the build is over
         with torch.cuda.stream(other):
             if release:
                 del arrays

@@ -68,6 +68,13 @@ except AttributeError:  # pragma: no cover - older torch
     _raw_stream = None
 
 
+# from_dataset copies device arrays of up to this many bytes in all.  Larger ones are
+# read where they are, and it waits for the build before it returns, which takes the
+# next call's 40 us of host work out of the build's shadow: about what copying this
+# much takes (back to back, 14 MB of events: 117 us copied, 148 in place; 112 MB: 190
+# and 210; 254 MB: 366 and 338).
+_ADOPT_COPY_BYTES = 128 << 20
+
 _WS_SIZES: dict = {}
 
 
@@ -405,30 +412,38 @@ class TemporalGraph:
         self._build_starts.append(n0)
         self._build_n = n1
 
-    def _build_adopt(self, src: Tensor, dst: Tensor, time: Tensor, feat: Optional[Tensor], call: int) -> bool:
+    def _build_adopt(self, src: Tensor, dst: Tensor, time: Tensor, feat: Optional[Tensor],
+                     call: int) -> Optional[bool]:
         """Take the events of advance() calls of ``call`` events each as the event
-        buffers of an empty graph, without copying device arrays that already have
-        the buffers' layout: for a caller that freezes the graph and waits for the
-        build before it returns, since until then the build reads the arrays where
-        they are, and whoever owns them may reuse them on any stream.  False, with
-        nothing taken, where advance() would refuse one of the calls."""
+        buffers of an empty graph, in as few copies as their layout asks for.  None,
+        with nothing taken, where advance() would refuse one of the calls; else
+        whether a buffer is the caller's own memory, which the build then reads where
+        it is: whoever owns it may reuse it on any stream, so the caller of this must
+        freeze the graph and wait for the build before it returns.  Small arrays are
+        copied, and freeze_csr()'s host round trip comes after those copies."""
         n = int(src.shape[0])
         if dst.shape[0] < n or time.shape[0] < n or (feat is not None and feat.shape[0] < n):
-            return False
-        arrays = [x[:n].detach().reshape(-1) for x in (src, dst, time)]
-        if n == 0 or any(x.shape[0] != n for x in arrays):
-            return False
-        if feat is not None:
-            feat = self._feat_in(feat[:n], n)
+            return None
+        given = {"src": src, "dst": dst, "time": time}
+        given = {k: x[:n].detach().reshape(-1) for k, x in given.items()}
+        if n == 0 or any(x.shape[0] != n for x in given.values()):
+            return None
         dev = self.device
-        self._build = {"src": _as(arrays[0], torch.int64, dev), "dst": _as(arrays[1], torch.int64, dev),
-                       "time": _as(arrays[2], torch.float64, dev)}
-        if feat is not None and self.edge_feat_dim > 0:
-            self._build["feat"] = feat.detach()
+        bufs = {k: _as(x, torch.float64 if k == "time" else torch.int64, dev) for k, x in given.items()}
+        if feat is not None:
+            rows = self._feat_in(feat[:n], n)
+            if self.edge_feat_dim > 0:
+                given["feat"], bufs["feat"] = feat, rows.detach()
+        own = [k for k, x in bufs.items() if x.data_ptr() != given[k].data_ptr()]
+        in_place = len(own) < len(bufs)
+        if in_place and sum(x.numel() * x.element_size() for x in bufs.values()) <= _ADOPT_COPY_BYTES:
+            bufs = {k: x if k in own else x.clone() for k, x in bufs.items()}
+            in_place = False
+        self._build = bufs
         self._build_starts = range(0, n, call)
         self._build_n = n
         self._num_edges = n
-        return True
+        return in_place
 
     def freeze_csr(self) -> None:
         """Build the frozen CSR on the device from the pre-freeze events
@@ -730,15 +745,15 @@ class TemporalGraph:
         graph = cls(num_nodes, edge_feat_dim=d_edge, device=device, **kwargs)
         chunk = 10000
         n = src.shape[0]
-        # all the calls' events at once, frozen where they are: 157,474 events with
-        # 172-d rows went through 82 copies and took 580 us with the freeze, 200 this
-        # way (157 without the wait, with the next call's host work beside the build)
-        if cls.advance is TemporalGraph.advance and graph._build_adopt(src, dst, time, edge_feat, chunk):
+        # all the calls' events at once: 157,474 events with 172-d rows went through 82
+        # copies and took 580 us with the freeze, 190 this way
+        in_place = graph._build_adopt(src, dst, time, edge_feat, chunk) if cls.advance is TemporalGraph.advance else None
+        if in_place is not None:
             try:
                 graph.freeze_csr()
             finally:
-                # the arrays are the caller's again, to refill or release on any stream
-                torch.cuda.current_stream(graph.device).synchronize()
+                if in_place:  # the arrays are the caller's again, to refill or release on any stream
+                    torch.cuda.current_stream(graph.device).synchronize()
             return graph
         for s in range(0, n, chunk):
             e = min(s + chunk, n)
