@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kThreads) void csr_scan_final(const ScanPart* __res
 // event's own segment from the bitmap, and writes the entries at their positions.  Times
 // and call starts are read for the marks once: the segments partition the events,
 // and the positions are a permutation, whatever the arrays hold, also where
-// another stream writes them meanwhile.  8M events in runs of three take 13 + 91 us, the keys
+// another stream writes them meanwhile.  8M events in runs of three take 13 + 4 + 82 us, the keys
 // and records of the next steps included (448 MB; before, marks, a device-wide scan
 // of them, segment starts, the order and the node keys took eight launches and 230 us).
 constexpr int kSegItems = 8;
